@@ -1,0 +1,62 @@
+"""GPU parity of the BF16 / F16 GEMM on the 16-bit matrix cores (vgx_qgemm with a workspace, used by
+ops.qlinear from 8 activation rows on) against the fp64 oracle.
+
+Bar: the fp32 accumulation bound at the one-row GEMV's relative term (2e-6).  The pieces hold 24 (BF16)
+and about 22 (F16) bits of the activations, 2^-22 at most, a tenth of it."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import codec, linalg
+from vault_amd import ops, vlt3
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dt", [codec.BF16, codec.F16])
+@pytest.mark.parametrize("rows,cols,batch,epi", [
+    (13, 32, 8, "store"), (2, 64, 65, "swiglu"), (257, 96, 63, "accum"), (1030, 1536, 129, "store"),
+    (1536, 8960, 64, "accum"), (640, 2048, 1000, "swiglu"), (256, 256, 9, "edge"), (70, 512, 40, "strided")])
+def test_wgemm_matches_oracle(dev, dt, rows, cols, batch, epi):
+    """Tile edges (256 weight rows, 64 activation rows), one K block, K splits with a short last one, every
+    epilogue; "edge": weights and rows of extreme magnitudes (fp16 subnormals, rows of 1e-30 .. 1e30) and
+    non-finite activations; "strided": rows at an odd float offset and stride."""
+    rng = np.random.default_rng(rows + cols + batch)
+    mk = lambda seed: vlt3.quantize(dt, np.random.default_rng(seed).standard_normal((rows, cols)).astype(np.float32)
+                                    * (1e-5 if epi == "edge" else 0.05))  # noqa: E731
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    if epi == "edge":
+        x *= (10.0 ** np.linspace(-30, 30, batch)).astype(np.float32)[:, None]
+        x[4, 7], x[5, 9] = np.inf, np.nan
+    if epi == "strided":
+        buf = torch.zeros(batch * (cols + 3) + 1, device=dev)
+        xt = buf[1:].view(batch, cols + 3)[:, :cols]
+        xt.copy_(torch.from_numpy(x))
+    else:
+        xt = torch.from_numpy(x).to(dev)
+    if epi == "swiglu":
+        g, u = mk(1), mk(2)
+        w = ops.QWeight.gateup_from_blocks(dt, rows, cols, g, u, dev)
+        h = ops.qlinear_swiglu(w, xt).cpu().numpy().astype(np.float64)
+        gf, uf = codec.decode(dt, g, rows, cols), codec.decode(dt, u, rows, cols)
+        gg, uu = linalg.gemv(gf, x), linalg.gemv(uf, x)
+        ref = linalg.swiglu(gg, uu)
+        tol = 1.1 * np.abs(uu) * linalg.gemv_bound(gf, x, dt) + np.abs(gg) * linalg.gemv_bound(uf, x, dt) + \
+            1e-6 * np.abs(ref) + 1e-30
+        assert np.all(np.abs(h - ref) <= tol), float((np.abs(h - ref) / tol).max())
+        return
+    raw = mk(3)
+    w, wf = ops.QWeight.from_blocks(dt, rows, cols, raw, dev), codec.decode(dt, raw, rows, cols)
+    bias = rng.standard_normal(rows).astype(np.float32) if epi != "edge" else None
+    y0 = rng.standard_normal((batch, rows)).astype(np.float32)
+    y = ops.qlinear(w, xt, bias=torch.from_numpy(bias).to(dev) if bias is not None else None,
+                    out=torch.from_numpy(y0).to(dev) if epi == "accum" else None, accumulate=epi == "accum")
+    y = y.cpu().numpy().astype(np.float64)
+    keep = np.isfinite(x).all(axis=1)
+    ref = linalg.gemv(wf, x[keep], bias) + (y0[keep] if epi == "accum" else 0.0)
+    tol = linalg.gemv_bound(wf, x[keep], dt) + np.abs(ref) * 2e-7
+    err = np.abs(y[keep] - ref)
+    assert np.all(err <= tol), float((err / tol).max())
+    if epi == "edge":
+        nz = wf[:, 7] != 0
+        assert np.all(np.isinf(y[4][nz])) and np.all(np.isnan(y[4][~nz])) and np.all(np.isnan(y[5]))

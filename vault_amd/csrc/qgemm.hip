@@ -52,9 +52,12 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // so 2^-k is a normal float; a row holding an infinity or a NaN is not scaled (k = 0), so that it
 // reaches the outputs as it would unsplit.
 // Inside every group of four, elements 1 and 2 trade places (stored order 0, 2, 1, 3): the K-slot
-// order of the tiled kernel's weight fragments, whose Q4_0 nibble pairs come out of a word that way.
+// order of the tiled kernel's weight fragments, whose Q4_0 nibble pairs come out of a word that way;
+// with NATURAL (F16 weights, wgemm_tile_kernel) they stay in place, and a non-finite element gets a zero
+// lo, so that an infinity reaches the outputs as one.
 // One workgroup of 256 threads per activation row.
 constexpr int kXsplitRegs = 20;   // float4 per thread kept in registers: rows of up to 20480 elements
+template <bool NATURAL = false>
 __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x, int64_t ldx,
                                                       const float *__restrict__ lnw, float eps, int cols,
                                                       uint16_t *__restrict__ xh, uint16_t *__restrict__ xl,
@@ -126,6 +129,15 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x
             v.x = g.x * (v.x * inv); v.y = g.y * (v.y * inv); v.z = g.z * (v.z * inv); v.w = g.w * (v.w * inv);
         }
         v.x *= sc; v.y *= sc; v.z *= sc; v.w *= sc;
+        if constexpr (NATURAL) {
+            const uint32_t h01 = pack_f16x2(v.x, v.y), h23 = pack_f16x2(v.z, v.w);
+            const auto hp = __builtin_bit_cast(vgx_f16x2_t, h01), hq = __builtin_bit_cast(vgx_f16x2_t, h23);
+            auto rest = [](float e, _Float16 h) { return __builtin_isfinite(e) ? e - (float)h : 0.0f; };
+            *reinterpret_cast<uint2 *>(xh + b * cols + 4 * i) = make_uint2(h01, h23);
+            *reinterpret_cast<uint2 *>(xl + b * cols + 4 * i) =
+                make_uint2(pack_f16x2(rest(v.x, hp[0]), rest(v.y, hp[1])), pack_f16x2(rest(v.z, hq[0]), rest(v.w, hq[1])));
+            return;
+        }
         // stored order 0, 2, 1, 3
         const uint32_t h02 = pack_f16x2(v.x, v.z), h13 = pack_f16x2(v.y, v.w);
         const auto hp = __builtin_bit_cast(vgx_f16x2_t, h02), hq = __builtin_bit_cast(vgx_f16x2_t, h13);
@@ -662,7 +674,8 @@ __global__ __launch_bounds__(256, 3) void qgemm_tile_dma_kernel(const uint8_t *_
 }
 
 // ---------------------------------------------------------------------------------------------
-// F32 / BF16 / F16 weights (the segment scorer's fc1, F32 and BF16 model files) for many activation
+// F32 weights (the segment scorer's fc1, F32 model files), and BF16 / F16 weights of callers without a
+// workspace or past wgemm_tile_kernel's buffer ranges, for many activation
 // rows, 16-bit elements widened exactly to fp32 as they are fetched: fp32 MFMA
 // (v_mfma_f32_16x16x4_f32), so products and sums stay fp32 as in the reference.  A workgroup of 4
 // waves owns 64 weight rows x 64 activation rows (each wave 32 x 32 as 2 x 2 tiles); per 32-wide
@@ -790,6 +803,12 @@ __global__ __launch_bounds__(256) void f32gemm_tile_kernel(const void *__restric
         }
     }
 }
+
+}  // namespace
+
+#include "wgemm.h"
+
+namespace {
 
 // ---------------------------------------------------------------------------------------------
 // Decode batches (up to 64 activation rows): one launch without the split pre-pass.  Each workgroup
@@ -2405,6 +2424,62 @@ int split_proj_launch(int dtype, const void *wp, int64_t rows, int64_t cols, con
     return ks;
 }
 
+// BF16 / F16 weights on wgemm_tile_kernel: planes, per-row scales, K-split partials.
+constexpr int kWgTM = 256, kWgTN = 64, kWgNS = 2;
+// K splits: as many as fit 512 workgroups (one round at two per CU), at least 8 blocks each.
+inline int wgemm_ksplit(int64_t n_rq, int64_t batch, int nblk) {
+    const int64_t tiles = (n_rq + kWgTM / 4 - 1) / (kWgTM / 4) * ((batch + kWgTN - 1) / kWgTN);
+    int64_t ks = 512 / tiles;
+    ks = std::min<int64_t>(ks, std::min<int64_t>(kMaxKSplit, nblk / 8));
+    return (int)std::max<int64_t>(1, ks);
+}
+inline int64_t wgemm_bytes(int64_t batch, int64_t n_rq, int nblk) {
+    const int64_t cols = (int64_t)nblk * QK;
+    return 3 * split_plane_bytes(batch, cols) + (batch * 4 + 255) / 256 * 256 +
+           part_bytes(wgemm_ksplit(n_rq, batch, nblk), batch, n_rq * 4);
+}
+
+template <int WDT>
+int wgemm_launch(const void *w_packed, int64_t rows, int64_t n_rq, int nblk, const float *x, int64_t ldx, int64_t batch,
+                 const float *bias, float *y, int64_t ldy, int epilogue, void *workspace, hipStream_t st) {
+    const int cols = nblk * QK;
+    const int64_t pb = split_plane_bytes(batch, cols);
+    char *const ws = static_cast<char *>(workspace);
+    auto *xs = reinterpret_cast<uint16_t *>(ws);
+    float *xsc = nullptr;
+    if constexpr (WDT == VGX_BF16) {
+        const int64_t n4 = batch * (cols / 4);
+        hipLaunchKernelGGL(xsplit_bf16x3_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, x, ldx, cols, n4, xs,
+                           pb / 2);
+    } else {
+        xsc = reinterpret_cast<float *>(ws + 3 * pb);
+        hipLaunchKernelGGL(xsplit_kernel<true>, dim3((unsigned)batch), dim3(256), 0, st, x, ldx, nullptr, 0.0f, cols, xs,
+                           xs + pb / 2, xsc);
+    }
+    VGX_CHECK_LAUNCH();
+    auto *part = reinterpret_cast<float *>(ws + 3 * pb + (batch * 4 + 255) / 256 * 256);
+    const int ks = wgemm_ksplit(n_rq, batch, nblk), kper = (nblk + ks - 1) / ks;
+    const dim3 grid((unsigned)((n_rq + kWgTM / 4 - 1) / (kWgTM / 4)), (unsigned)((batch + kWgTN - 1) / kWgTN), (unsigned)ks);
+    const auto *w = static_cast<const uint8_t *>(w_packed);
+#define VGX_WG(EPI, SP)                                                                                            hipLaunchKernelGGL((wgemm_tile_kernel<WDT, EPI, SP, kWgTM, kWgTN, kWgNS>), grid, dim3(kWgTM * kWgTN / 64), 0, st, w,                        n_rq, nblk, rows, xs, pb / 2, xsc, batch, bias, y, ldy, part, kper)
+    if (ks > 1) VGX_WG(EPI_STORE, true);
+    else if (epilogue == VGX_EPI_SWIGLU) VGX_WG(EPI_SWIGLU, false);
+    else if (epilogue == VGX_EPI_ACCUM) VGX_WG(EPI_ACCUM, false);
+    else VGX_WG(EPI_STORE, false);
+#undef VGX_WG
+    VGX_CHECK_LAUNCH();
+    if (ks > 1) {
+        if (epilogue == VGX_EPI_SWIGLU)
+            reduce_launch<EPI_SWIGLU>(part, ks, batch, n_rq * 4, rows, bias, y, ldy, nullptr, cols, 0.0f, st);
+        else if (epilogue == VGX_EPI_ACCUM)
+            reduce_launch<EPI_ACCUM>(part, ks, batch, n_rq * 4, rows, bias, y, ldy, nullptr, cols, 0.0f, st);
+        else
+            reduce_launch<EPI_STORE>(part, ks, batch, n_rq * 4, rows, bias, y, ldy, nullptr, cols, 0.0f, st);
+        VGX_CHECK_LAUNCH();
+    }
+    return VGX_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -2418,7 +2493,9 @@ int64_t vgx_qgemm_workspace_bytes(int64_t batch, int64_t rows, int64_t cols, int
     // the weight dtype is not an argument: the larger of the Q4_0 and Q8_0 layouts
     const int64_t sq4 = small_bytes(batch, rows_p / 4, (int)(cols / QK), VGX_Q4_0);
     const int64_t sq8 = small_bytes(batch, rows_p / 4, (int)(cols / QK), VGX_Q8_0);
-    return batch <= kSmallMaxBatch ? std::max(big, std::max(sq4, sq8)) : big;
+    // ... nor is it for the BF16 / F16 layout
+    const int64_t all = std::max(big, wgemm_bytes(batch, rows_p / 4, (int)(cols / QK)));
+    return batch <= kSmallMaxBatch ? std::max(all, std::max(sq4, sq8)) : all;
 }
 
 int vgx_qgemm(int dtype, const void *w_packed, int64_t rows, int64_t cols, const float *x, int64_t ldx, int64_t batch,
@@ -2439,6 +2516,20 @@ int vgx_qgemm(int dtype, const void *w_packed, int64_t rows, int64_t cols, const
     const int64_t n_rq = rows4(rows_packed) / 4;
     if (dtype == VGX_F32 || dtype == VGX_BF16 || dtype == VGX_F16) {
         if (norm_w) return VGX_E_ARG;                 // plain weights: no fused RMSNorm on this path
+        // 16-bit weights on the 16-bit matrix cores when the caller brought the workspace and the operands
+        // fit the DMA's buffer ranges; without one (it is optional here) on the fp32 MFMA.  Gate/up | down
+        // of BF16 files at 8, 40, 333, 1024 rows: 107 -> 25, 108 -> 33, 243 -> 76, 591 -> 184 us | 472 ->
+        // 24, 474 -> 28, 462 -> 53, 467 -> 107 us: ahead at every batch size this entry takes
+        const int64_t pbytes = 3 * split_plane_bytes(batch, cols);
+        if (dtype != VGX_F32 && workspace && (uintptr_t)workspace % 256 == 0 &&
+            workspace_bytes >= wgemm_bytes(batch, n_rq, nblk) && n_rq * nblk * 256 < ((int64_t)1 << 31) &&
+            pbytes < ((int64_t)1 << 31)) {
+            if (dtype == VGX_BF16)
+                return wgemm_launch<VGX_BF16>(w_packed, rows, n_rq, nblk, x, ldx, batch, bias, y, ldy, epilogue, workspace,
+                                              (hipStream_t)stream);
+            return wgemm_launch<VGX_F16>(w_packed, rows, n_rq, nblk, x, ldx, batch, bias, y, ldy, epilogue, workspace,
+                                         (hipStream_t)stream);
+        }
         const void *wf = w_packed;
         const dim3 grid((unsigned)((n_rq + kFT / 4 - 1) / (kFT / 4)), (unsigned)((batch + kFT - 1) / kFT));
         const bool vec = ((uintptr_t)x & 15) == 0 && ldx % 4 == 0;
@@ -2573,7 +2664,7 @@ int vgx_qgemm(int dtype, const void *w_packed, int64_t rows, int64_t cols, const
     auto *xl = reinterpret_cast<uint16_t *>(wsb + pb);
     auto *xsc = reinterpret_cast<float *>(wsb + 2 * pb);
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(xsplit_kernel, dim3((unsigned)batch), dim3(256), 0, st, x, ldx, norm_w, eps, (int)cols, xh, xl,
+    hipLaunchKernelGGL(xsplit_kernel<false>, dim3((unsigned)batch), dim3(256), 0, st, x, ldx, norm_w, eps, (int)cols, xh, xl,
                        xsc);
     VGX_CHECK_LAUNCH();
     auto *part = reinterpret_cast<float *>(wsb + split_bytes(batch, cols));

@@ -177,7 +177,10 @@ def _gemv(w: QWeight, x: torch.Tensor, out: Optional[torch.Tensor], epi: int, bi
     if B >= GEMM_MIN_ROWS and (w.dtype in (Q8_0, Q4_0) or w.dtype in ELEM_BYTES):
         lib = L.load()
         need = int(lib.vgx_qgemm_workspace_bytes(B, w.rows, w.cols, epi))
-        ws = gemm_workspace(x.device).get(need)
+        # BF16 / F16 weights take no tickets: scratch of their own per call (stream-ordered), so that calls on
+        # several streams stay independent
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if w.dtype in (BF16, F16) else \
+            gemm_workspace(x.device).get(need)
         L.check(lib.vgx_qgemm(w.dtype, w.packed.data_ptr(), w.rows, w.cols, x2.data_ptr(), x2.stride(0), B, _ptr(nw),
                               float(eps), _ptr(bias), y2.data_ptr(), y2.stride(0), epi, ws.data_ptr(), ws.numel(),
                               _stream(x.device)), "vgx_qgemm")
