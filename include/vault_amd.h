@@ -261,8 +261,8 @@ typedef struct {
     int bias_run;
 } vgx_attn_block;
 
-/* Prefill attention on bf16 MFMA (kv_dtype VGX_BF16, or VGX_F32 whose K / V enter the MFMAs as bf16
- * hi + lo pairs; q_dtype VGX_F32 (hi + lo) or VGX_BF16; D = 128; H/G in {1, 2, 4, 6, 8}) for up to 8
+/* Prefill attention on bf16 MFMA (kv_dtype VGX_BF16, or VGX_F32 whose K / V enter the MFMAs as three
+ * bf16 pieces; q_dtype VGX_F32 (hi + lo) or VGX_BF16; D = 128; H/G in {1, 2, 4, 6, 8}) for up to 8
  * query blocks in one launch: out = softmax(q k^T * scale) v per query head h over kv group h / (H/G),
  * key tiles wholly in a query tile's causal future skipped.  out_dtype VGX_F32, or VGX_BF16 (the fp32
  * result rounded to nearest even, for bf16 callers).
@@ -270,6 +270,14 @@ typedef struct {
  * chunk-recurrent prefill (:2064-2093). */
 int vgx_attn_prefill(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_block *blocks, int n_blocks, int64_t H,
                      int64_t G, int64_t D, float scale, void *stream);
+
+/* vgx_attn_prefill with the planes of its fp32 K / V in a workspace (16-byte aligned, vgx_attn_prefill_planes_bytes of
+ * the same blocks): each 64 keys of a kv group as fp16 hi + lo under a power of two, converted once per call instead
+ * of by every workgroup that reads them (a smaller workspace, and bf16 K / V, run as vgx_attn_prefill). */
+int64_t vgx_attn_prefill_planes_bytes(int kv_dtype, const vgx_attn_block *blocks, int n_blocks, int64_t H, int64_t G);
+int vgx_attn_prefill_planes(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_block *blocks, int n_blocks,
+                            int64_t H, int64_t G, int64_t D, float scale, void *workspace, int64_t workspace_bytes,
+                            void *stream);
 
 /* vgx_attn_prefill with a workspace (16-byte aligned, at least vgx_attn_prefill_workspace_bytes(H, G)
  * bytes): a launch of few query tiles (a chunk of the chunk-recurrent prefill) splits each tile's keys

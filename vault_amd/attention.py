@@ -6,7 +6,7 @@ src/vault_v3_model.py:812-863: q (B, H, L, D) post-RoPE, k / v (B, G, L, D) post
 i-1, causally to chunk i, and for i >= 2 to the first n_sink tokens re-rotated to the virtual
 positions (i-1)W - n_sink + j (clamped at 0; :805-809).  The attention runs in the MFMA prefill
 kernel (vgx_attn_prefill) in the dtype of k / v, as the reference's SDPA runs in its input dtype:
-bf16 K / V as they are, fp32 K / V as three bf16 pieces each (fp32-level results); other float
+bf16 K / V as they are, fp32 K / V as scaled fp16 hi + lo or three bf16 pieces (fp32-level results); other float
 dtypes take the fp32 path.  The sink keys are re-rotated on the GPU (vgx_rope_rotate) in fp32 with
 float32 angles, the reference's rope_cos_sin arithmetic (:777-782), and stored once in the K / V
 dtype (the reference rotates bf16 keys in bf16 arithmetic, :790-794, which rounds three times).

@@ -19,19 +19,27 @@
 //   O^T (dims x queries) += V^T P^T    A = V^T from LDS, B = P^T straight from the S^T accumulators
 //                                      as a bf16 hi + lo pair (two MFMAs): 8-bit probabilities alone
 //                                      exceed the bf16 attention bound when few keys carry the weight.
-// Staging.  bf16 K / V at 4 or more heads per group are copied into LDS by LDS DMA (buffer loads that
-// write LDS, no registers or VALU involved), double-buffered in 128-key tiles: the next tile's loads
+// Staging.  K / V are copied into LDS by LDS DMA (buffer loads that
+// write LDS, no registers or VALU involved), double-buffered in 128-key tiles (fp32: 64-key tiles of the
+// fp16 planes below): the next tile's loads
 // leave right after the barrier that publishes the current one.  Both tiles keep the rows as they are
 // in memory (256 bytes per key), each 16-byte piece p of row r stored at slot p ^ (r & 15), so the
 // 16-byte K reads of 16 rows and the transposed V reads stay free of bank conflicts; the V^T operand
 // comes from ds_read_b64_tr_b16, which hands lane i of a 16-lane group element i % 4 of the 8-byte
 // pieces that lanes i / 4 + 4 k address (k = 0..3): lane lq addresses key 4 lg + lq / 4, dims
-// 16 dt + 4 (lq % 4) .. + 3, and receives dim 16 dt + lq of keys 4 lg .. 4 lg + 3.  Otherwise (fp32
-// K / V, one or two heads per group) each tile is loaded into registers during the previous tile's
-// math and stored into LDS, K as is (padded rows), V transposed.
-// bf16 K and V stay bf16 end to end (no conversions in the staging loop): MFMA throughput is abundant
-// here, VALU issue is what bounds the kernel.  fp32 K and V (an fp32 state read in place) are staged
-// as three bf16 planes (hi, mid, lo: 24 significant bits, the whole fp32 mantissa), and the fp32
+// 16 dt + 4 (lq % 4) .. + 3, and receives dim 16 dt + lq of keys 4 lg .. 4 lg + 3.
+// bf16 K and V stay bf16 end to end.  fp32 K and V with a workspace for planes: kv_pair_kernel writes them once per call as
+// fp16 hi + lo planes (22 bits or more) under a power of two per 64 keys and kv group; queries (a power of two
+// each) and probabilities are split the same way, and each product keeps hi x hi, hi x lo and lo x hi.  The K scale
+// multiplies the scores; the V scale enters the weights' exponent, so it is part of the running max, and is taken out
+// of the sum.  Three MFMAs per product and no conversions in the tile loop instead of six and the staging below:
+// two sequences of 2500 at 12 / 2 heads 359 -> 186 us, at 4 / 4 heads 887 -> 174 (what is left there is the host's
+// side of the call); relative error against 64 bits 4.4e-7 -> 3.5e-7.  At 3584 keys the kernel takes 76 us for 1024
+// queries (19.3 GFLOP, its MFMAs 23 us at peak): the chain scores -> softmax -> P V of three waves per SIMD and
+// 32 KB of LDS reads per wave and 32 keys bound it.
+// Without that workspace, for few keys, or with key ranges (vgx_attn_prefill_ws), each fp32 tile is loaded into registers during the previous tile's
+// math and stored into LDS as three bf16 planes (hi, mid, lo: 24 significant bits), K as is (padded rows), V
+// transposed; the fp32
 // queries and the probabilities are split the same way; each product keeps the six piece pairs of
 // order <= 2 (hi x hi, hi x mid, mid x hi, hi x lo, lo x hi, mid x mid) and drops those below 2^-24
 // of it, so scores and outputs carry fp32-level error (about 2^-22 relative) instead of the 2^-17 of
@@ -51,14 +59,14 @@ using namespace vgx;
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kKT = 64;             // keys per LDS tile
-constexpr int kKTDma = 128;         // keys per LDS tile of bf16 K / V staged by LDS DMA
 constexpr int kD = 128;             // head dim (the kernel is specialised for 128)
 constexpr int kKRow = kD + 8;       // LDS row of K, bf16 (16 bytes of padding)
 constexpr int kMaxBlocks = 8;
 constexpr float kNegBig = -1.0e30f;
+constexpr int kPrefillMaxSplit = 4;   // key ranges per query tile
 constexpr float kLazyMax = 8.0f;    // log2 of the largest unnormalised probability
 
 typedef short v4i16_t __attribute__((ext_vector_type(4)));
@@ -76,11 +84,18 @@ __device__ __forceinline__ T sel4(int i, T a0, T a1, T a2, T a3) {
 }
 
 struct RunArgs {
-    const void *k;     // bf16 or fp32 rows
-    const void *v;
+    const void *k;     // bf16 or fp32 rows; fp16 pair planes: the run's first plane
+    const void *v;     // fp16 pair planes: the run's PairScale entries
     int64_t len;
-    int64_t rstride;   // elements between consecutive keys
+    int64_t rstride;   // elements between consecutive keys; fp16 pair planes: rows per kv group
     int64_t gstride;   // elements between kv groups
+};
+
+// Power-of-two scales of kPairKeys keys of one kv group: the plane holds 2^-log2 x the value.
+constexpr int kPairKeys = 64;
+struct PairScale {
+    float k;           // 2^log2 of the K rows
+    float v_log2;      // log2 of the V rows' scale
 };
 
 struct BlockArgs {
@@ -94,6 +109,7 @@ struct BlockArgs {
     int64_t causal_base;
     int n_runs;
     int tile0;         // first workgroup index of this block
+    int src;           // its index in the caller's list
     RunArgs run[4];
     // optional bias on run bias_run: query t of head h adds bias[t * bias_ldq + head_row[h] * bias_rstride
     // + j] to its score with key j of that run (head_row[h] < 0: none)
@@ -120,19 +136,112 @@ struct PrefillArgs {
 // the running max and sum.
 __host__ __device__ constexpr int prefill_slot_floats(int waves, int nqt) { return waves * nqt * (8 * 256 + 32); }
 
-template <int GRP, bool QSPLIT, int NQT, bool KF, int QW, bool DMA>
+constexpr float kPairBoost = 6.0f;  // log2 of the weights' scale: at most 2^(kLazyMax + 6) < 65504 in fp16
+
+template <bool F16>
+__device__ __forceinline__ f32x4_t mfma16(bf16x8_t x, bf16x8_t y, f32x4_t c) {
+    if constexpr (F16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, x), __builtin_bit_cast(f16x8_t, y), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ float exp2i(int k) { return __uint_as_float((uint32_t)(k + 127) << 23); }   // |k| <= 126
+__device__ __forceinline__ float finite_abs(float x) { return __builtin_isfinite(x) ? fabsf(x) : 0.0f; }
+// k with 2^k mx in [2^14, 2^15), at most 100 (also for mx = 0: zero V rows then weigh nothing against the others in
+// the running max), so that sums of 2^k x probabilities stay in the fp32 range
+__device__ __forceinline__ int pair_exponent(float mx) { return min(100, 14 + 127 - (int)(__float_as_uint(mx) >> 23)); }
+// hi = fp16(a, b), lo = fp16(a - hi_a, b - hi_b) (0 where a, b is not finite)
+__device__ __forceinline__ void split_f16x2(float a, float b, uint32_t &hi, uint32_t &lo) {
+    hi = pack_f16x2(a, b);
+    const auto h = __builtin_bit_cast(vgx_f16x2_t, hi);
+    lo = pack_f16x2(a - (float)h[0], b - (float)h[1]);
+}
+
+// fp32 K / V runs as fp16 hi + lo planes, so that the attention kernel stages them by LDS DMA and needs three
+// MFMAs per product instead of the six of three bf16 planes.  Each kPairKeys keys of a kv group share a power
+// of two per operand (largest |element| in [2^14, 2^15)), so both pieces are normal fp16 numbers for every
+// element above 2^-28 of it, and the pair holds 22 bits or more.  A non-finite element is left
+// out of the scale and keeps its value in hi with a zero lo.
+struct PairRun {
+    const float *k, *v;
+    int64_t len, rstride, gstride;
+    int64_t rows;              // len rounded up to kPairKeys
+    uint16_t *planes;          // K hi, K lo, V hi, V lo: [G][rows][kD] each
+    PairScale *scale;          // [G][rows / kPairKeys]
+    int wg0;                   // first workgroup of this run
+};
+constexpr int kMaxPairRuns = 4 * kMaxBlocks;
+struct PairArgs {
+    PairRun run[kMaxPairRuns];
+    int n_runs, G;
+};
+
+// One workgroup per (kPairKeys keys, kv group, K or V).
+__global__ __launch_bounds__(256) void kv_pair_kernel(PairArgs a) {
+    int ri = 0;
+    for (int i = 1; i < a.n_runs; ++i)
+        if (a.run[i].wg0 <= (int)blockIdx.x) ri = i;
+    const PairRun &R = a.run[ri];
+    const int local = blockIdx.x - R.wg0, isv = local & 1, g = (local >> 1) % a.G, grp = (local >> 1) / a.G;
+    const int64_t j0 = (int64_t)grp * kPairKeys;
+    const float *src = (isv ? R.v : R.k) + (int64_t)g * R.gstride;
+    constexpr int IT = kPairKeys * kD / 4 / 256;
+    const int col = threadIdx.x & 31, row0 = threadIdx.x >> 5;
+    float4 x[IT];
+    float mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+        const int64_t j = j0 + row0 + 8 * i;
+        x[i] = j < R.len ? *reinterpret_cast<const float4 *>(src + j * R.rstride + 4 * col) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+        mx = fmaxf(fmaxf(fmaxf(mx, finite_abs(x[i].x)), finite_abs(x[i].y)), fmaxf(finite_abs(x[i].z), finite_abs(x[i].w)));
+    for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
+    __shared__ float wm[4];
+    if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    const int k = pair_exponent(fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3])));
+    const float sc = exp2i(k);
+    if (threadIdx.x == 0) {
+        PairScale *e = R.scale + (int64_t)g * (R.rows / kPairKeys) + grp;
+        if (isv) e->v_log2 = (float)-k;
+        else e->k = exp2i(-k);
+    }
+    const int64_t ps = (int64_t)a.G * R.rows * kD;
+    uint16_t *hp = R.planes + (isv ? 2 * ps : 0) + ((int64_t)g * R.rows + j0) * kD;
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+        const int row = row0 + 8 * i;
+        uint2 hi, lo;
+        const float e[4] = {x[i].x * sc, x[i].y * sc, x[i].z * sc, x[i].w * sc};
+        split_f16x2(e[0], e[1], hi.x, lo.x);
+        split_f16x2(e[2], e[3], hi.y, lo.y);
+        if (!__builtin_isfinite(e[0])) lo.x &= 0xFFFF0000u;
+        if (!__builtin_isfinite(e[1])) lo.x &= 0xFFFFu;
+        if (!__builtin_isfinite(e[2])) lo.y &= 0xFFFF0000u;
+        if (!__builtin_isfinite(e[3])) lo.y &= 0xFFFFu;
+        *reinterpret_cast<uint2 *>(hp + row * kD + 4 * col) = hi;
+        *reinterpret_cast<uint2 *>(hp + ps + row * kD + 4 * col) = lo;
+    }
+}
+
+template <int GRP, bool QSPLIT, int NQT, bool KF, int QW, bool DMA, int KT>
 __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs a) {
     constexpr int kQTile = 16 * NQT * QW;
-    // keys per LDS tile (fp32 K / V: 32, staged as three bf16 planes)
-    constexpr int KT = KF ? 32 : (DMA ? kKTDma : kKT);
+    constexpr bool PAIR = KF && DMA;                // fp32 K / V as the fp16 hi + lo planes of kv_pair_kernel
     constexpr int VROW = KT + 8;                    // LDS row of V^T, bf16 (16 bytes of padding)
-    constexpr int NP = KF ? 3 : 1;                  // bf16 planes per K / V operand
-    constexpr int NQP = QSPLIT ? (KF ? 3 : 2) : 1;  // bf16 pieces per query
-    constexpr int NPP = KF ? 3 : 2;                 // bf16 pieces per probability
-    constexpr int ORD = KF ? 2 : 1;                 // products of pieces i x j kept when i + j <= ORD
-    constexpr int ESZ = KF ? 4 : 2;                 // bytes per K / V element in memory
-    static_assert(!DMA || !KF, "LDS DMA stages bf16 K / V as they are");
-    __shared__ __align__(16) uint16_t ks[DMA ? 2 * 2 * KT * kD : NP * KT * kKRow];   // DMA: [stage][K, V][key][dim]
+    constexpr int NP = PAIR ? 2 : KF ? 3 : 1;       // 16-bit planes per K / V operand
+    constexpr int NQP = QSPLIT ? (KF && !PAIR ? 3 : 2) : 1;  // 16-bit pieces per query
+    constexpr int NPP = KF && !PAIR ? 3 : 2;        // 16-bit pieces per probability
+    constexpr int ORD = KF && !PAIR ? 2 : 1;        // products of pieces i x j kept when i + j <= ORD
+    constexpr int ESZ = KF && !PAIR ? 4 : 2;        // bytes per staged K / V element in memory
+    constexpr int STAGE_E = 2 * NP * KT * kD;       // DMA: elements per stage
+    constexpr int CH = 32;                          // keys per softmax step
+    static_assert(KF || DMA, "bf16 K / V are staged by LDS DMA");
+    static_assert(!PAIR || KT == kPairKeys, "one scale per tile");
+    __shared__ __align__(16) uint16_t ks[DMA ? 2 * STAGE_E : NP * KT * kKRow];   // DMA: [stage][K planes, V planes][key][dim]
     __shared__ __align__(16) uint16_t vt[DMA ? 8 : NP * kD * VROW];
 
     // XCD-aware order: consecutive tiles (same block and group, neighbouring queries, same keys; the
@@ -158,36 +267,77 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
     // Q^T fragments (bf16): query t0 + 16 qt + lq, dims 32 kc + 8 lg .. + 7; fp32 queries as NQP
     // pieces: hi = bf16(q), then bf16 of what is left (lo, or mid and lo).
     bf16x8_t qf[NQP][NQT][4];
+    float qinv[NQT];                                // PAIR: 2^-k of the query's scale
+    if constexpr (PAIR) {
+        // fp16 pieces of the query scaled by a power of two (largest element in [2^14, 2^15))
 #pragma unroll
-    for (int qt = 0; qt < NQT; ++qt) {
-        const int64_t t = tw + qt * 16 + lq;
+        for (int qt = 0; qt < NQT; ++qt) {
+            const int64_t t = tw + qt * 16 + lq;
+            float e[4][8], mx = 0.0f;
 #pragma unroll
-        for (int kc = 0; kc < 4; ++kc) {
-            const int d0 = kc * 32 + lg * 8;
-            uint32_t pw[NQP][4];
-            if (t < B.n_q) {
-                if constexpr (!QSPLIT) {
-                    const uint4 w = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(B.q) + t * B.ldq + h * B.q_hstride + d0);
-                    pw[0][0] = w.x; pw[0][1] = w.y; pw[0][2] = w.z; pw[0][3] = w.w;
-                } else {
-                    const float *qp = static_cast<const float *>(B.q) + t * B.ldq + h * B.q_hstride + d0;
+            for (int kc = 0; kc < 4; ++kc) {
+                const int64_t at = t * B.ldq + h * B.q_hstride + kc * 32 + lg * 8;
+                if (t >= B.n_q) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) e[kc][i] = 0.0f;
+                } else if constexpr (QSPLIT) {
+                    const float *qp = static_cast<const float *>(B.q) + at;
                     const float4 x0 = reinterpret_cast<const float4 *>(qp)[0], x1 = reinterpret_cast<const float4 *>(qp)[1];
-                    const float e[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+                    e[kc][0] = x0.x; e[kc][1] = x0.y; e[kc][2] = x0.z; e[kc][3] = x0.w;
+                    e[kc][4] = x1.x; e[kc][5] = x1.y; e[kc][6] = x1.z; e[kc][7] = x1.w;
+                } else {
+                    const uint4 w = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(B.q) + at);
+                    const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        if constexpr (NQP == 3) split3_bf16x2(e[2 * i], e[2 * i + 1], pw[0][i], pw[1][i], pw[2][i]);
-                        else split_bf16x2(e[2 * i], e[2 * i + 1], pw[0][i], pw[NQP - 1][i]);
-                    }
+                    for (int i = 0; i < 8; ++i) e[kc][i] = bf16_bits_to_float(ww[i / 2] >> (i & 1) * 16);
                 }
-            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) mx = fmaxf(mx, finite_abs(e[kc][i]));
+            }
+            const int k = pair_exponent(xor32_max(xor16_max(mx)));
+            qinv[qt] = exp2i(-k);
+            const float sc = exp2i(k);
+#pragma unroll
+            for (int kc = 0; kc < 4; ++kc) {
+                uint32_t hi[4], lo[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) split_f16x2(e[kc][2 * i] * sc, e[kc][2 * i + 1] * sc, hi[i], lo[i]);
+                qf[0][qt][kc] = __builtin_bit_cast(bf16x8_t, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+                if constexpr (NQP == 2) qf[NQP - 1][qt][kc] = __builtin_bit_cast(bf16x8_t, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+            }
+        }
+    } else {
+#pragma unroll
+        for (int qt = 0; qt < NQT; ++qt) {
+            const int64_t t = tw + qt * 16 + lq;
+#pragma unroll
+            for (int kc = 0; kc < 4; ++kc) {
+                const int d0 = kc * 32 + lg * 8;
+                uint32_t pw[NQP][4];
+                if (t < B.n_q) {
+                    if constexpr (!QSPLIT) {
+                        const uint4 w = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(B.q) + t * B.ldq + h * B.q_hstride + d0);
+                        pw[0][0] = w.x; pw[0][1] = w.y; pw[0][2] = w.z; pw[0][3] = w.w;
+                    } else {
+                        const float *qp = static_cast<const float *>(B.q) + t * B.ldq + h * B.q_hstride + d0;
+                        const float4 x0 = reinterpret_cast<const float4 *>(qp)[0], x1 = reinterpret_cast<const float4 *>(qp)[1];
+                        const float e[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            if constexpr (NQP == 3) split3_bf16x2(e[2 * i], e[2 * i + 1], pw[0][i], pw[1][i], pw[2][i]);
+                            else split_bf16x2(e[2 * i], e[2 * i + 1], pw[0][i], pw[NQP - 1][i]);
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int pp = 0; pp < NQP; ++pp)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) pw[pp][i] = 0;
+                }
 #pragma unroll
                 for (int pp = 0; pp < NQP; ++pp)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) pw[pp][i] = 0;
+                    qf[pp][qt][kc] = __builtin_bit_cast(bf16x8_t, make_uint4(pw[pp][0], pw[pp][1], pw[pp][2], pw[pp][3]));
             }
-#pragma unroll
-            for (int pp = 0; pp < NQP; ++pp)
-                qf[pp][qt][kc] = __builtin_bit_cast(bf16x8_t, make_uint4(pw[pp][0], pw[pp][1], pw[pp][2], pw[pp][3]));
         }
     }
 
@@ -207,13 +357,19 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
     const int64_t cbase = B.causal_base;
     int64_t rlen[4];
     const char *rkp[4], *rvp[4];
-    int rrs[4];
+    int rrs[4];                                    // PAIR: bytes between planes / 256
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const RunArgs &R = B.run[i];
         int64_t n = i < n_runs ? R.len : 0;
         if (i == n_runs - 1 && cbase >= 0) n = min(n, cbase + t0 + kQTile);   // the rest is in every query's future
         rlen[i] = n;
+        if constexpr (PAIR) {
+            rkp[i] = static_cast<const char *>(R.k) + (int64_t)g * R.rstride * (kD * 2);
+            rvp[i] = static_cast<const char *>(R.v) + (int64_t)g * (R.rstride / kPairKeys) * sizeof(PairScale);
+            rrs[i] = (int)R.rstride * a.G;
+            continue;
+        }
         rkp[i] = static_cast<const char *>(R.k) + (int64_t)g * R.gstride * ESZ;
         rvp[i] = static_cast<const char *>(R.v) + (int64_t)g * R.gstride * ESZ;
         rrs[i] = (int)R.rstride * ESZ;             // bytes between consecutive keys
@@ -253,7 +409,27 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
             }
         }
     };
+    PairScale tsc{1.0f, 0.0f};                     // PAIR: the scales of the tile in flight
     auto issue = [&](int r, int64_t j0, int buf) {
+        if constexpr (PAIR) {
+            constexpr int RB = kD * 2;
+            const char *p0 = sel4(r, rkp[0], rkp[1], rkp[2], rkp[3]) + j0 * RB;
+            const int64_t ps = (int64_t)sel4(r, rrs[0], rrs[1], rrs[2], rrs[3]) * RB;
+            const int lim = (int)min<int64_t>(run_len(r) - j0, KT);
+            tsc = reinterpret_cast<const PairScale *>(sel4(r, rvp[0], rvp[1], rvp[2], rvp[3]))[j0 / kPairKeys];
+            dma_rsrc_t rs[4];                       // K hi, K lo, V hi, V lo
+#pragma unroll
+            for (int p = 0; p < 4; ++p) rs[p] = dma_rsrc(p0 + p * ps, (uint32_t)(lim * RB));
+            uint8_t *base = reinterpret_cast<uint8_t *>(ks) + buf * (STAGE_E * 2);
+            const int sub = lane >> 4, slot = lane & 15;
+            for (int i = wave; i < KT / 4; i += NT / 64) {      // 4 rows of each plane
+                const int row = 4 * i + sub;
+                const uint32_t off = (uint32_t)(row * RB + ((slot ^ (row & 15)) << 4));
+#pragma unroll
+                for (int p = 0; p < 4; ++p) dma16(rs[p], off, base + (p * KT + 4 * i) * RB);
+            }
+            return;
+        }
         const int64_t n = run_len(r);
         const int rs = sel4(r, rrs[0], rrs[1], rrs[2], rrs[3]);
         const char *kb = sel4(r, rkp[0], rkp[1], rkp[2], rkp[3]) + j0 * rs;
@@ -274,18 +450,14 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
         for (int i = 0; i < KIT; ++i) {
             const int c = tid + i * NT;
             if (c >= KCH) continue;
-            if constexpr (!KF) {
-                *reinterpret_cast<uint4 *>(ks + (c >> 4) * kKRow + (c & 15) * 8) = kreg[i];
-            } else {
-                // four fp32 of row c / 32 -> bf16 hi, mid and lo (planes 0, 1, 2)
-                uint2 hw, mw, lw;
-                split3_bf16x2(__uint_as_float(kreg[i].x), __uint_as_float(kreg[i].y), hw.x, mw.x, lw.x);
-                split3_bf16x2(__uint_as_float(kreg[i].z), __uint_as_float(kreg[i].w), hw.y, mw.y, lw.y);
-                uint16_t *kp = ks + (c / CPR) * kKRow + (c % CPR) * 4;
-                *reinterpret_cast<uint2 *>(kp) = hw;
-                *reinterpret_cast<uint2 *>(kp + KT * kKRow) = mw;
-                *reinterpret_cast<uint2 *>(kp + 2 * KT * kKRow) = lw;
-            }
+            // four fp32 of row c / 32 -> bf16 hi, mid and lo (planes 0, 1, 2)
+            uint2 hw, mw, lw;
+            split3_bf16x2(__uint_as_float(kreg[i].x), __uint_as_float(kreg[i].y), hw.x, mw.x, lw.x);
+            split3_bf16x2(__uint_as_float(kreg[i].z), __uint_as_float(kreg[i].w), hw.y, mw.y, lw.y);
+            uint16_t *kp = ks + (c / CPR) * kKRow + (c % CPR) * 4;
+            *reinterpret_cast<uint2 *>(kp) = hw;
+            *reinterpret_cast<uint2 *>(kp + KT * kKRow) = mw;
+            *reinterpret_cast<uint2 *>(kp + 2 * KT * kKRow) = lw;
         }
 #pragma unroll
         for (int i = 0; i < VIT; ++i) {
@@ -294,25 +466,14 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
             const int rp = c % (KT / 2), cc = c / (KT / 2);
             const uint32_t a0[4] = {vreg[i][0].x, vreg[i][0].y, vreg[i][0].z, vreg[i][0].w};
             const uint32_t a1[4] = {vreg[i][1].x, vreg[i][1].y, vreg[i][1].z, vreg[i][1].w};
-            if constexpr (!KF) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    // dims 8 cc + 2 e and + 1 of keys 2 rp, 2 rp + 1: one 4-byte word each
-                    *reinterpret_cast<uint32_t *>(vt + (cc * 8 + 2 * e) * VROW + 2 * rp) =
-                        (a0[e] & 0xFFFFu) | (a1[e] << 16);
-                    *reinterpret_cast<uint32_t *>(vt + (cc * 8 + 2 * e + 1) * VROW + 2 * rp) =
-                        (a0[e] >> 16) | (a1[e] & 0xFFFF0000u);
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    // dim 4 cc + e of keys 2 rp, 2 rp + 1: the hi, mid and lo words
-                    uint32_t hw, mw, lw;
-                    split3_bf16x2(__uint_as_float(a0[e]), __uint_as_float(a1[e]), hw, mw, lw);
-                    *reinterpret_cast<uint32_t *>(vt + (cc * 4 + e) * VROW + 2 * rp) = hw;
-                    *reinterpret_cast<uint32_t *>(vt + kD * VROW + (cc * 4 + e) * VROW + 2 * rp) = mw;
-                    *reinterpret_cast<uint32_t *>(vt + 2 * kD * VROW + (cc * 4 + e) * VROW + 2 * rp) = lw;
-                }
+            for (int e = 0; e < 4; ++e) {
+                // dim 4 cc + e of keys 2 rp, 2 rp + 1: the hi, mid and lo words
+                uint32_t hw, mw, lw;
+                split3_bf16x2(__uint_as_float(a0[e]), __uint_as_float(a1[e]), hw, mw, lw);
+                *reinterpret_cast<uint32_t *>(vt + (cc * 4 + e) * VROW + 2 * rp) = hw;
+                *reinterpret_cast<uint32_t *>(vt + kD * VROW + (cc * 4 + e) * VROW + 2 * rp) = mw;
+                *reinterpret_cast<uint32_t *>(vt + 2 * kD * VROW + (cc * 4 + e) * VROW + 2 * rp) = lw;
             }
         }
     };
@@ -346,6 +507,7 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
     }
     if (todo == 0) r = n_runs;
     int buf = 0;
+    float kscale = 1.0f, vlog = 0.0f, vinv = 1.0f;  // PAIR: 2^log2 of the tile's K, log2 and 2^-log2 of its V
     if constexpr (DMA) {
         if (r < n_runs) issue(r, j0, 0);
     } else {
@@ -365,6 +527,11 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
             // this tile's loads landed (each wave waits for its own, the barrier for every wave's), and
             // every wave is done with the other stage: the next tile's loads go there
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if constexpr (PAIR) {
+                kscale = tsc.k * sl2;
+                vlog = tsc.v_log2;
+                vinv = __builtin_amdgcn_exp2f(-vlog);
+            }
             if (rn < n_runs) issue(rn, jn, buf ^ 1);
         } else {
             __syncthreads();
@@ -372,45 +539,44 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
             __syncthreads();
             if (rn < n_runs) fetch(rn, jn);
         }
-        const uint8_t *kst = reinterpret_cast<const uint8_t *>(ks) + buf * (2 * KT * kD * 2);
-        const uint8_t *vst = kst + KT * kD * 2;
-        auto scores = [&](int c, f32x4_t (&sc)[NQT][2]) {
+        const uint8_t *kst = reinterpret_cast<const uint8_t *>(ks) + buf * (STAGE_E * 2);
+        const uint8_t *vst = kst + NP * KT * kD * 2;
+        constexpr int NS = CH / 16;                 // 16-key score tiles per step
+        auto scores = [&](int c, f32x4_t (&sc)[NQT][NS]) {
 #pragma unroll
-            for (int qt = 0; qt < NQT; ++qt) {
-                sc[qt][0] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                sc[qt][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            }
+            for (int qt = 0; qt < NQT; ++qt)
+#pragma unroll
+                for (int s = 0; s < NS; ++s) sc[qt][s] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int kc = 0; kc < 4; ++kc) {
 #pragma unroll
                 for (int pk = 0; pk < NP; ++pk) {        // K plane: hi (then, fp32 K, mid and lo)
-                    bf16x8_t a0, a1;
-                    if constexpr (DMA) {
-                        // rows c + lq, c + 16 + lq: 16-byte piece kc * 4 + lg stored at slot piece ^ (row & 15)
-                        const int so = ((kc * 4 + lg) ^ lq) << 4;
-                        a0 = *reinterpret_cast<const bf16x8_t *>(kst + (c + lq) * (kD * 2) + so);
-                        a1 = *reinterpret_cast<const bf16x8_t *>(kst + (c + 16 + lq) * (kD * 2) + so);
-                    } else {
-                        const uint16_t *kp = ks + pk * KT * kKRow;
-                        a0 = *reinterpret_cast<const bf16x8_t *>(kp + (c + lq) * kKRow + kc * 32 + lg * 8);
-                        a1 = *reinterpret_cast<const bf16x8_t *>(kp + (c + 16 + lq) * kKRow + kc * 32 + lg * 8);
+                    bf16x8_t af[NS];
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) {
+                        const int row = c + 16 * s + lq;
+                        if constexpr (DMA)          // 16-byte piece kc * 4 + lg stored at slot piece ^ (row & 15)
+                            af[s] = *reinterpret_cast<const bf16x8_t *>(kst + (pk * KT + row) * (kD * 2) +
+                                                                        (((kc * 4 + lg) ^ lq) << 4));
+                        else
+                            af[s] = *reinterpret_cast<const bf16x8_t *>(ks + (pk * KT + row) * kKRow + kc * 32 + lg * 8);
                     }
 #pragma unroll
                     for (int qp = 0; qp < NQP; ++qp) {
-                        if (pk + qp > ORD) continue;      // below 2^-(8 (ORD + 1)) of the product
+                        if (pk + qp > ORD) continue;      // below 2^-(8 (ORD + 1)) of the product (PAIR: 2^-24)
 #pragma unroll
-                        for (int qt = 0; qt < NQT; ++qt) {
-                            sc[qt][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, qf[qp][qt][kc], sc[qt][0], 0, 0, 0);
-                            sc[qt][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, qf[qp][qt][kc], sc[qt][1], 0, 0, 0);
-                        }
+                        for (int s = 0; s < NS; ++s)
+#pragma unroll
+                            for (int qt = 0; qt < NQT; ++qt)
+                                sc[qt][s] = mfma16<PAIR>(af[s], qf[qp][qt][kc], sc[qt][s]);
                     }
                 }
             }
         };
-        auto finish = [&](int c, f32x4_t (&sc)[NQT][2]) {
-            bf16x8_t pf[NPP][NQT];
-            // 32-key chunk fully visible to all 32 queries: no per-score mask
-            const bool full = j0 + c + 32 <= n && (!causal || j0 + c + 31 <= cbase + tw);
+        auto finish = [&](int c, f32x4_t (&sc)[NQT][NS]) {
+            bf16x8_t pf[NPP][NQT][NS / 2];
+            // step fully visible to all of the wave's queries: no per-score mask
+            const bool full = j0 + c + CH <= n && (!causal || j0 + c + CH - 1 <= cbase + tw);
             // the biased run of a biased head: its bias (log2 units) is added to the chunk's scores
             const bool biased = brow != nullptr && r == B.bias_run;   // wave-uniform
             // key index relative to the causal limit of query t0 (fits in 32 bits)
@@ -418,39 +584,36 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
             const int klim = (int)(n - (j0 + c));
 #pragma unroll
             for (int qt = 0; qt < NQT; ++qt) {
-                float v[8];
+                float v[4 * NS];
+                float ssc = sl2;
+                if constexpr (PAIR) ssc = kscale * qinv[qt];
                 if (full) {
 #pragma unroll
-                    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) v[kt * 4 + i] = sc[qt][kt][i] * sl2;
+                    for (int i = 0; i < 4 * NS; ++i) v[i] = sc[qt][i / 4][i % 4] * ssc;
                 } else {
 #pragma unroll
-                    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int kk = kt * 16 + lg * 4 + i;       // key within the 32-key chunk
-                            const bool vis = kk < klim && (!causal || kbase + kk <= qt * 16 + lq);
-                            v[kt * 4 + i] = vis ? sc[qt][kt][i] * sl2 : -INFINITY;
-                        }
+                    for (int i = 0; i < 4 * NS; ++i) {
+                        const int kk = i / 4 * 16 + lg * 4 + i % 4;        // key within the step
+                        const bool vis = kk < klim && (!causal || kbase + kk <= qt * 16 + lq);
+                        v[i] = vis ? sc[qt][i / 4][i % 4] * ssc : -INFINITY;
+                    }
                 }
                 if (biased) {
                     const float *bq = brow + min(tw + qt * 16 + lq, B.n_q - 1) * B.bias_ldq;
 #pragma unroll
-                    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int64_t key = j0 + c + kt * 16 + lg * 4 + i;
-                            if (key < n) v[kt * 4 + i] += bq[key] * 1.4426950408889634f;   // -inf stays -inf
-                        }
+                    for (int i = 0; i < 4 * NS; ++i) {
+                        const int64_t key = j0 + c + i / 4 * 16 + lg * 4 + i % 4;
+                        if (key < n) v[i] += bq[key] * 1.4426950408889634f;   // -inf stays -inf
+                    }
                 }
                 float mt = v[0];
 #pragma unroll
-                for (int i = 1; i < 8; ++i) mt = fmaxf(mt, v[i]);
+                for (int i = 1; i < 4 * NS; ++i) mt = fmaxf(mt, v[i]);
                 mt = xor32_max(xor16_max(mt));
-                // The reference max m (log2 units) moves only when a score exceeds it by more than
-                // kLazyMax: probabilities then stay below 2^kLazyMax, and O and the sum are rescaled
-                // far less often than the running max changes.
+                if constexpr (PAIR) mt += vlog;
+                // The reference max m (log2 units; PAIR: of score + log2 of the V scale) moves only when a
+                // score exceeds it by more than kLazyMax: probabilities then stay below 2^kLazyMax, and O
+                // and the sum are rescaled far less often than the running max changes.
                 if (__ballot(mt > m[qt] + kLazyMax)) {
                     const float mn = fmaxf(m[qt], mt);
                     const float corr = __builtin_amdgcn_exp2f(m[qt] - mn);
@@ -459,58 +622,67 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
 #pragma unroll
                     for (int dt = 0; dt < 8; ++dt) o[qt][dt] *= corr;
                 }
-                const float mn = m[qt];
-                float ps = 0.0f, pv[8];
+                // PAIR: the weights carry the V scale and 2^kPairBoost, so that the lo pieces stay normal
+                const float mn = PAIR ? m[qt] - (vlog + kPairBoost) : m[qt];
+                float ps = 0.0f, pv[4 * NS];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
+                for (int i = 0; i < 4 * NS; ++i) {
                     pv[i] = __builtin_amdgcn_exp2f(v[i] - mn);
                     ps += pv[i];
                 }
-                uint32_t pw[NPP][4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if constexpr (NPP == 3) split3_bf16x2(pv[2 * i], pv[2 * i + 1], pw[0][i], pw[1][i], pw[2][i]);
-                    else split_bf16x2(pv[2 * i], pv[2 * i + 1], pw[0][i], pw[1][i]);
+                for (int s2 = 0; s2 < NS / 2; ++s2) {
+                    uint32_t pw[NPP][4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float x = pv[8 * s2 + 2 * i], y = pv[8 * s2 + 2 * i + 1];
+                        if constexpr (PAIR) split_f16x2(x, y, pw[0][i], pw[1][i]);
+                        else if constexpr (NPP == 3) split3_bf16x2(x, y, pw[0][i], pw[1][i], pw[2][i]);
+                        else split_bf16x2(x, y, pw[0][i], pw[1][i]);
+                    }
+#pragma unroll
+                    for (int pp = 0; pp < NPP; ++pp)
+                        pf[pp][qt][s2] =
+                            __builtin_bit_cast(bf16x8_t, make_uint4(pw[pp][0], pw[pp][1], pw[pp][2], pw[pp][3]));
                 }
-#pragma unroll
-                for (int pp = 0; pp < NPP; ++pp)
-                    pf[pp][qt] = __builtin_bit_cast(bf16x8_t, make_uint4(pw[pp][0], pw[pp][1], pw[pp][2], pw[pp][3]));
+                if constexpr (PAIR) ps *= vinv;
                 lsum[qt] += ps;
             }
 #pragma unroll
             for (int dt = 0; dt < 8; ++dt) {
 #pragma unroll
-                for (int pv_ = 0; pv_ < NP; ++pv_) {     // V plane: hi (then, fp32 V, mid and lo)
-                    bf16x8_t va;
-                    if constexpr (DMA) {
-                        // transposed reads of the row-major tile: lane lq of group lg addresses key
-                        // c + 4 lg + lq / 4, dims 16 dt + 4 (lq % 4) .. + 3, and receives dim 16 dt + lq of
-                        // keys c + 4 lg .. + 3 (then of the same keys + 16)
-                        const int row = c + lg * 4 + (lq >> 2);
-                        const int off = row * (kD * 2) + (((dt * 2 + ((lq & 3) >> 1)) ^ (row & 15)) << 4) + ((lq & 1) << 3);
-                        const v4i16_t lo = lds_read_tr16(vst + off), hi = lds_read_tr16(vst + off + 16 * (kD * 2));
-                        typedef short v8i16_t __attribute__((ext_vector_type(8)));
-                        const v8i16_t w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                        va = __builtin_bit_cast(bf16x8_t, w);
-                    } else {
-                        const uint16_t *vr = vt + pv_ * kD * VROW + (dt * 16 + lq) * VROW + c + lg * 4;
-                        const uint2 lo = *reinterpret_cast<const uint2 *>(vr);
-                        const uint2 hi = *reinterpret_cast<const uint2 *>(vr + 16);
-                        va = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
-                    }
+                for (int s2 = 0; s2 < NS / 2; ++s2)
 #pragma unroll
-                    for (int pp = 0; pp < NPP; ++pp) {
-                        if (pv_ + pp > ORD) continue;     // as for the scores
+                    for (int pv_ = 0; pv_ < NP; ++pv_) {     // V plane: hi (then mid and lo, PAIR: lo)
+                        bf16x8_t va;
+                        if constexpr (DMA) {
+                            // transposed reads of the row-major tile: lane lq of group lg addresses key
+                            // c + 4 lg + lq / 4, dims 16 dt + 4 (lq % 4) .. + 3, and receives dim 16 dt + lq of
+                            // keys c + 4 lg .. + 3 (then of the same keys + 16)
+                            const int row = c + 32 * s2 + lg * 4 + (lq >> 2);
+                            const int off = (pv_ * KT + row) * (kD * 2) +
+                                            (((dt * 2 + ((lq & 3) >> 1)) ^ (row & 15)) << 4) + ((lq & 1) << 3);
+                            const v4i16_t lo = lds_read_tr16(vst + off), hi = lds_read_tr16(vst + off + 16 * (kD * 2));
+                            const v8i16_t w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                            va = __builtin_bit_cast(bf16x8_t, w);
+                        } else {
+                            const uint16_t *vr = vt + pv_ * kD * VROW + (dt * 16 + lq) * VROW + c + 32 * s2 + lg * 4;
+                            const uint2 lo = *reinterpret_cast<const uint2 *>(vr);
+                            const uint2 hi = *reinterpret_cast<const uint2 *>(vr + 16);
+                            va = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
+                        }
 #pragma unroll
-                        for (int qt = 0; qt < NQT; ++qt)
-                            o[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pf[pp][qt], o[qt][dt], 0, 0, 0);
+                        for (int pp = 0; pp < NPP; ++pp) {
+                            if (pv_ + pp > ORD) continue;     // as for the scores
+#pragma unroll
+                            for (int qt = 0; qt < NQT; ++qt) o[qt][dt] = mfma16<PAIR>(va, pf[pp][qt][s2], o[qt][dt]);
+                        }
                     }
-                }
             }
         };
-        for (int c = 0; c < KT && j0 + c < n; c += 32) {
+        for (int c = 0; c < KT && j0 + c < n; c += CH) {
             if (causal && j0 + c > cbase + tw + 16 * NQT - 1) break;   // wave-uniform: the wave's future
-            f32x4_t sc[NQT][2];
+            f32x4_t sc[NQT][NS];
             scores(c, sc);
             finish(c, sc);
         }
@@ -587,9 +759,9 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_merge_kernel(Prefi
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) {
         const int64_t t = tw + qt * 16 + lq;
-        float mp[4], lp[4], M = kNegBig;
+        float mp[kPrefillMaxSplit], lp[kPrefillMaxSplit], M = kNegBig;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+        for (int p = 0; p < kPrefillMaxSplit; ++p) {
             mp[p] = kNegBig;
             lp[p] = 0.0f;
             if (p < ns) {
@@ -600,9 +772,9 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_merge_kernel(Prefi
                 M = fmaxf(M, v.x);
             }
         }
-        float w[4], L = 0.0f;
+        float w[kPrefillMaxSplit], L = 0.0f;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+        for (int p = 0; p < kPrefillMaxSplit; ++p) {
             w[p] = p < ns ? __builtin_amdgcn_exp2f(mp[p] - M) : 0.0f;
             L += w[p] * lp[p];
         }
@@ -613,7 +785,7 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_merge_kernel(Prefi
         for (int dt = 0; dt < 8; ++dt) {
             float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
+            for (int p = 0; p < kPrefillMaxSplit; ++p) {
                 if (p >= ns) continue;
                 const float4 x = *reinterpret_cast<const float4 *>(slot0 + (int64_t)p * prefill_slot_floats(NWV, NQT) +
                                                                    (((wave * NQT + qt) * 8 + dt) * 64 + lane) * 4);
@@ -631,36 +803,109 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_merge_kernel(Prefi
     }
 }
 
-// Launch shape per K / V dtype and heads per group: NQT 16-query tiles per wave, QW waves per head, LDS
-// DMA staging.  At 4 and 6 heads per group a workgroup of 2 GRP waves of 16 queries (at most 168
-// registers, three waves per SIMD: one workgroup of 12 waves per CU at 6 heads) keeps more waves in
-// flight than GRP waves of 32 queries (226-256 registers, two per SIMD, 6 waves per CU), for the same
-// K / V tile per 32 queries.  Measured at L = 8192 (12 query / 2 KV heads, drop-in call): bf16 K / V
-// 333 -> 295 us with 2 x 6 waves of 16 queries, -> 264 us with the tiles staged by LDS DMA (64 keys),
-// -> 247 us with 128-key tiles; fp32 K / V 1082 -> 749 us with 2 x 6 waves.  Eight heads per group
-// keep 8 waves of 32 queries (16 waves would need <= 128 registers and spill), one and two the
-// register-staged 32-query waves.  A launch of fewer 2-wave-per-head workgroups than CUs (a 2048-query
-// chunk of the chunk-recurrent prefill at 2 KV heads: 128) runs one wave per head instead (narrow):
-// twice the workgroups over the CUs.
+// Launch shape per K / V kind and heads per group: QW waves of NQT 16-query tiles per head.  Waves of 16 queries
+// (at most 168 registers: three per SIMD) beat waves of 32 (226-256 registers, two), and a workgroup of 8-12 waves
+// shares each staged tile: 12 query / 2 KV heads at L = 8192, bf16: 333 -> 295 us with 2 x 6 waves of 16 instead of
+// 6 of 32, -> 247 us with 128-key tiles by LDS DMA.  One and two heads per group take 8 and 4 waves per head: a
+// 1024-query chunk over 2560 keys at 4 / 4 heads, bf16, 127 -> 43 us, at 8 / 4 104 -> 48 us against the one-wave
+// workgroups that staged V through registers (fp32 planes: 331 -> 53 us for 777 queries over 1901 keys at 4 / 4).  Eight heads per
+// group keep 8 waves of 32 bf16 queries (16 waves would need <= 128 registers and spill).
+// A launch of fewer workgroups than CUs takes half the waves per head (narrow), twice the workgroups.  With a
+// workspace the key ranges fill the CUs already, and the wide shape, which stages half the tiles per query, is ahead
+// while they do: the 1024-query bf16 chunk at 12 / 2 heads over 3584 keys (64 wide tiles x 4 ranges against 128 x 2)
+// 83 -> 68 us, 700 queries over 2236 (44 x 4) 56 -> 52; 400 (26) loses, 42 -> 50.  fp32 K / V with key ranges stay on
+// the in-place kernel and its shapes.
 constexpr int kPrefillNarrowBelow = 256;
-constexpr int prefill_nqt(int grp, bool kf) { return kf || grp == 4 || grp == 6 ? 1 : 2; }
-constexpr int prefill_qw(int grp, bool kf, bool narrow) {
-    return !narrow && (grp == 4 || grp == 6 || (kf && grp == 2)) ? 2 : 1;
+constexpr int kSplitNarrowBelow = 40;
+// Fewer keys than this in every block: the conversion's own launch costs more than the faster tiles give, and fp32
+// K / V are read in place.  12 / 2 heads, causal, in place | planes, us: 64 keys 14.5 | 18.1, 128 20.1 | 17.8, 200
+// 29.5 | 21.8, 512 60.1 | 35.8.
+constexpr int kPairMinKeys = 128;
+enum { kKvBf16 = 0, kKvF32 = 1, kKvPair = 2 };   // bf16, fp32 in place (three bf16 planes), fp32 as fp16 pair planes
+constexpr int prefill_nqt(int grp, int kv) { return kv == kKvBf16 && grp == 8 ? 2 : 1; }
+constexpr int prefill_qw(int grp, int kv, bool narrow) {
+    if (kv == kKvF32) return !narrow && (grp == 2 || grp == 4 || grp == 6) ? 2 : 1;
+    return (grp == 1 ? 8 : grp == 2 ? 4 : grp == 8 ? 1 : 2) / (narrow && grp != 8 ? 2 : 1);
 }
-constexpr bool prefill_dma(int grp, bool kf) { return !kf && grp >= 4; }
+// keys per LDS tile
+constexpr int prefill_kt(int kv) { return kv == kKvBf16 ? 128 : kv == kKvPair ? kPairKeys : 32; }
 
 // Key-range splits: with a workspace, a launch of fewer than kPrefillNarrowBelow workgroups (a
 // 1024-query chunk of the chunk-recurrent prefill at 2 KV heads: 128) splits each tile's keys into up to
 // four ranges, so that the launch fills the CUs; attn_prefill_merge_kernel then combines them.
-constexpr int kPrefillMaxSplit = 4;
+
 // Workspace bound: at most kPrefillNarrowBelow (tile, range) slots, each of at most 2 GRP waves x 2
-// 16-query tiles.
+// 16-query tiles (one head per group: 8 waves of one).
 inline int64_t prefill_ws_bytes(int grp) {
-    return (int64_t)kPrefillNarrowBelow * prefill_slot_floats(2 * grp, 2) * 4;
+    return (int64_t)kPrefillNarrowBelow * prefill_slot_floats(std::max(2 * grp, 4), 2) * 4;
+}
+
+// Launch shape of a call and, for fp32 K / V, the runs that kv_pair_kernel converts (runs over the same rows, as
+// two chunks share one, only once).
+struct PrefillPlan {
+    int kv = kKvBf16;
+    bool narrow = false;
+    int qtile = 0, n_split = 1, split_wgs = 0;
+    int64_t tiles = 0, bytes = 0, max_keys = 0;
+    PairArgs pair{};
+    int run_of[kMaxBlocks][4] = {};        // PAIR: block, run -> pair.run
+};
+
+PrefillPlan prefill_plan(int kv, const vgx_attn_block *blocks, int n_blocks, int64_t G, int grp, bool split) {
+    PrefillPlan p;
+    p.kv = kv;
+    auto count = [&](int q) {
+        int64_t t = 0;
+        for (int i = 0; i < n_blocks; ++i)
+            if (blocks[i].n_q > 0) t += (blocks[i].n_q + q - 1) / q * G;
+        return t;
+    };
+    const int wide = kv == kKvF32 ? 32 : 16 * prefill_nqt(grp, kv) * prefill_qw(grp, kv, false);
+    p.narrow = prefill_qw(grp, kv, false) > 1 && count(wide) < (split && kv != kKvF32 ? kSplitNarrowBelow : kPrefillNarrowBelow);
+    p.qtile = 16 * prefill_nqt(grp, kv) * prefill_qw(grp, kv, p.narrow);   // queries per workgroup
+    p.tiles = count(p.qtile);
+    if (split && p.tiles > 0 && p.tiles < kPrefillNarrowBelow)
+        p.n_split = (int)std::min<int64_t>(kPrefillMaxSplit, kPrefillNarrowBelow / p.tiles);
+    if (kv != kKvPair) return p;
+    PairArgs &pa = p.pair;
+    pa.G = (int)G;
+    for (int i = 0; i < n_blocks; ++i) {
+        int64_t keys = 0;
+        for (int r = 0; blocks[i].n_q > 0 && r < blocks[i].n_runs; ++r) {
+            keys += blocks[i].runs[r].len;
+            const vgx_kv_run &R = blocks[i].runs[r];
+            int u = 0;
+            while (u < pa.n_runs && (pa.run[u].k != R.k || pa.run[u].v != R.v || pa.run[u].rstride != R.row_stride ||
+                                     pa.run[u].gstride != R.group_stride))
+                ++u;
+            if (u == pa.n_runs) {
+                PairRun &n = pa.run[pa.n_runs++];
+                n.k = static_cast<const float *>(R.k);
+                n.v = static_cast<const float *>(R.v);
+                n.rstride = R.row_stride;
+                n.gstride = R.group_stride;
+            }
+            pa.run[u].len = std::max(pa.run[u].len, R.len);
+            p.run_of[i][r] = u;
+        }
+        p.max_keys = std::max(p.max_keys, keys);
+    }
+    for (int u = 0; u < pa.n_runs; ++u) {
+        PairRun &n = pa.run[u];
+        n.rows = (n.len + kPairKeys - 1) / kPairKeys * kPairKeys;
+        n.planes = reinterpret_cast<uint16_t *>(p.bytes);        // offsets; the call adds the workspace
+        p.bytes += 4 * G * n.rows * kD * 2;
+        n.scale = reinterpret_cast<PairScale *>(p.bytes);
+        p.bytes += (G * (n.rows / kPairKeys) * (int64_t)sizeof(PairScale) + 255) / 256 * 256;
+        n.wg0 = p.split_wgs;
+        p.split_wgs += (int)(n.rows / kPairKeys * G * 2);
+    }
+    return p;
 }
 
 int attn_prefill_impl(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_block *blocks, int n_blocks, int64_t H,
-                      int64_t G, int64_t D, float scale, void *workspace, int64_t workspace_bytes, void *stream) {
+                      int64_t G, int64_t D, float scale, bool split, void *workspace, int64_t workspace_bytes,
+                      void *stream) {
     if (kv_dtype != VGX_BF16 && kv_dtype != VGX_F32) return VGX_E_DTYPE;
     if (out_dtype != VGX_F32 && out_dtype != VGX_BF16) return VGX_E_DTYPE;
     const int oel = out_dtype == VGX_BF16 ? 2 : 4;
@@ -672,19 +917,12 @@ int attn_prefill_impl(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_b
     if (D != kD) return VGX_E_LIMIT;
     const int grp = (int)(H / G);
     if (grp != 1 && grp != 2 && grp != 4 && grp != 6 && grp != 8) return VGX_E_LIMIT;
-    const bool kf = kv_dtype == VGX_F32;
-    int64_t wide_tiles = 0;
-    for (int i = 0; i < n_blocks; ++i)
-        if (blocks[i].n_q > 0) wide_tiles += (blocks[i].n_q + 31) / 32 * G;
-    const bool narrow = prefill_qw(grp, kf, false) > 1 && wide_tiles < kPrefillNarrowBelow;
-    const int qtile = 16 * prefill_nqt(grp, kf) * prefill_qw(grp, kf, narrow);   // queries per workgroup
     PrefillArgs a{};
     a.H = (int)H;
     a.G = (int)G;
     a.scale_log2 = scale * 1.4426950408889634f;
     a.q_bf16 = q_dtype == VGX_BF16;
     a.o_bf16 = out_dtype == VGX_BF16;
-    int64_t tiles = 0;
     int nb = 0;
     for (int i = 0; i < n_blocks; ++i) {
         const vgx_attn_block &b = blocks[i];
@@ -706,7 +944,6 @@ int attn_prefill_impl(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_b
         B.n_q = b.n_q;
         B.causal_base = b.causal_base;
         B.n_runs = b.n_runs;
-        B.tile0 = (int)tiles;
         if (b.bias) {
             if (!b.bias_head_row || b.bias_run < 0 || b.bias_run >= b.n_runs) return VGX_E_ARG;
             if (b.bias_ldq < 0 || b.bias_rstride < 0) return VGX_E_SIZE;
@@ -732,40 +969,82 @@ int attn_prefill_impl(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_b
             B.run[r].gstride = R.group_stride;
             n_keys += R.len;
         }
+        B.src = i;
         if (b.causal_base >= 0 && b.causal_base + 1 > b.runs[b.n_runs - 1].len) return VGX_E_SIZE;
         if (n_keys == 0) return VGX_E_SIZE;
-        tiles += (b.n_q + qtile - 1) / qtile * G;
         ++nb;
     }
     if (nb == 0) return VGX_OK;
-    if (tiles > 0x7FFFFFFF) return VGX_E_LIMIT;
+    PrefillPlan p = prefill_plan(kv_dtype == VGX_F32 ? kKvF32 : kKvBf16, blocks, n_blocks, G, grp, split);
+    if (p.tiles > 0x7FFFFFFF) return VGX_E_LIMIT;
+    const bool ws_ok = workspace && (uintptr_t)workspace % 16 == 0;
+    if (split && !(ws_ok && workspace_bytes >= prefill_ws_bytes(grp))) {
+        // refused for a launch of few 32-query tiles (16-query ones where two waves share a head), else unsplit
+        int64_t t32 = 0, t16 = 0;
+        for (int i = 0; i < nb; ++i) {
+            t32 += (a.blk[i].n_q + 31) / 32 * G;
+            t16 += (a.blk[i].n_q + 15) / 16 * G;
+        }
+        const bool small = kv_dtype == VGX_F32 ? p.tiles < kPrefillNarrowBelow
+                                               : (grp == 4 || grp == 6 ? t16 : t32) < kPrefillNarrowBelow;
+        if (small) return workspace_bytes < prefill_ws_bytes(grp) ? VGX_E_ARENA : VGX_E_ALIGN;
+        p.n_split = 1;
+    }
+    // fp32 K / V through the pair planes when the workspace holds them
+    if (kv_dtype == VGX_F32 && ws_ok && !split) {
+        const PrefillPlan pp = prefill_plan(kKvPair, blocks, n_blocks, G, grp, false);
+        if (pp.bytes <= workspace_bytes && pp.bytes < ((int64_t)1 << 37) && pp.max_keys >= kPairMinKeys)
+            p = pp;                                               // (32-bit workgroup and row counts)
+    }
+    int64_t tiles = 0;
+    for (int i = 0; i < nb; ++i) {
+        a.blk[i].tile0 = (int)tiles;
+        tiles += (a.blk[i].n_q + p.qtile - 1) / p.qtile * G;
+    }
     a.n_blocks = nb;
     a.n_tiles = (int)tiles;
-    a.n_split = 1;
-    if (workspace != nullptr && tiles < kPrefillNarrowBelow) {
-        if (workspace_bytes < prefill_ws_bytes(grp)) return VGX_E_ARENA;
-        if ((uintptr_t)workspace % 16) return VGX_E_ALIGN;
-        a.n_split = (int)std::min<int64_t>(kPrefillMaxSplit, kPrefillNarrowBelow / tiles);
-        a.ws = static_cast<float *>(workspace);
+    a.n_split = p.n_split;
+    a.ws = static_cast<float *>(workspace);
+    if (p.kv == kKvPair) {
+        char *const ws = static_cast<char *>(workspace);
+        for (int u = 0; u < p.pair.n_runs; ++u) {
+            PairRun &n = p.pair.run[u];
+            n.planes = reinterpret_cast<uint16_t *>(ws + reinterpret_cast<int64_t>(n.planes));
+            n.scale = reinterpret_cast<PairScale *>(ws + reinterpret_cast<int64_t>(n.scale));
+        }
+        for (int i = 0; i < nb; ++i)
+            for (int r = 0; r < a.blk[i].n_runs; ++r) {
+                const PairRun &n = p.pair.run[p.run_of[a.blk[i].src][r]];
+                a.blk[i].run[r].k = n.planes;
+                a.blk[i].run[r].v = n.scale;
+                a.blk[i].run[r].rstride = n.rows;
+            }
+        hipLaunchKernelGGL(kv_pair_kernel, dim3((unsigned)p.split_wgs), dim3(256), 0, (hipStream_t)stream, p.pair);
+        VGX_CHECK_LAUNCH();
     }
+    const bool narrow = p.narrow;
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid((unsigned)(tiles * a.n_split));
-#define VGX_PREFILL_SHAPE(G_, S_, KF_, N_)                                                                   \
-    do {                                                                                                     \
-        hipLaunchKernelGGL((attn_prefill_kernel<G_, S_, prefill_nqt(G_, KF_), KF_, prefill_qw(G_, KF_, N_),    \
-                                                prefill_dma(G_, KF_)>),                                        \
-                           grid, dim3(64 * G_ * prefill_qw(G_, KF_, N_)), 0, st, a);                           \
-        if (a.n_split > 1)                                                                                   \
-            hipLaunchKernelGGL((attn_prefill_merge_kernel<G_, prefill_nqt(G_, KF_), prefill_qw(G_, KF_, N_)>),  \
-                               dim3((unsigned)tiles), dim3(64 * G_ * prefill_qw(G_, KF_, N_)), 0, st, a);      \
+#define VGX_PREFILL_SHAPE(G_, S_, KV_, N_)                                                                    \
+    do {                                                                                                      \
+        hipLaunchKernelGGL((attn_prefill_kernel<G_, S_, prefill_nqt(G_, KV_), KV_ != kKvBf16, prefill_qw(G_, KV_, N_), \
+                                                KV_ != kKvF32, prefill_kt(KV_)>),  \
+                           grid, dim3(64 * G_ * prefill_qw(G_, KV_, N_)), 0, st, a);                           \
+        if (a.n_split > 1)                                                                                    \
+            hipLaunchKernelGGL((attn_prefill_merge_kernel<G_, prefill_nqt(G_, KV_), prefill_qw(G_, KV_, N_)>),  \
+                               dim3((unsigned)tiles), dim3(64 * G_ * prefill_qw(G_, KV_, N_)), 0, st, a);      \
     } while (0)
-#define VGX_PREFILL_GO(G_, S_)                                                                               \
-    do {                                                                                                     \
-        if (kf) {                                                                                            \
-            if (narrow) VGX_PREFILL_SHAPE(G_, S_, true, true); else VGX_PREFILL_SHAPE(G_, S_, true, false);  \
-        } else {                                                                                             \
-            if (narrow) VGX_PREFILL_SHAPE(G_, S_, false, true); else VGX_PREFILL_SHAPE(G_, S_, false, false);\
-        }                                                                                                    \
+#define VGX_PREFILL_KV(G_, S_, KV_) \
+    if (narrow) VGX_PREFILL_SHAPE(G_, S_, KV_, true); else VGX_PREFILL_SHAPE(G_, S_, KV_, false)
+#define VGX_PREFILL_GO(G_, S_)                                     \
+    do {                                                           \
+        if (p.kv == kKvPair) {                                     \
+            VGX_PREFILL_KV(G_, S_, kKvPair);                       \
+        } else if (p.kv == kKvF32) {                               \
+            VGX_PREFILL_KV(G_, S_, kKvF32);                        \
+        } else {                                                   \
+            VGX_PREFILL_KV(G_, S_, kKvBf16);                       \
+        }                                                          \
     } while (0)
 #define VGX_PREFILL_GRP(S_)                      \
     switch (grp) {                               \
@@ -782,6 +1061,7 @@ int attn_prefill_impl(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_b
     }
 #undef VGX_PREFILL_GRP
 #undef VGX_PREFILL_GO
+#undef VGX_PREFILL_KV
 #undef VGX_PREFILL_SHAPE
     VGX_CHECK_LAUNCH();
     return VGX_OK;
@@ -793,7 +1073,7 @@ extern "C" {
 
 int vgx_attn_prefill(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_block *blocks, int n_blocks, int64_t H,
                      int64_t G, int64_t D, float scale, void *stream) {
-    return attn_prefill_impl(kv_dtype, q_dtype, out_dtype, blocks, n_blocks, H, G, D, scale, nullptr, 0, stream);
+    return attn_prefill_impl(kv_dtype, q_dtype, out_dtype, blocks, n_blocks, H, G, D, scale, false, nullptr, 0, stream);
 }
 
 int64_t vgx_attn_prefill_workspace_bytes(int64_t H, int64_t G) {
@@ -802,11 +1082,35 @@ int64_t vgx_attn_prefill_workspace_bytes(int64_t H, int64_t G) {
     return prefill_ws_bytes((int)(H / G));
 }
 
+int64_t vgx_attn_prefill_planes_bytes(int kv_dtype, const vgx_attn_block *blocks, int n_blocks, int64_t H, int64_t G) {
+    const int64_t base = vgx_attn_prefill_workspace_bytes(H, G);
+    if (base < 0) return base;
+    if (kv_dtype != VGX_F32) return 0;
+    if (!blocks) return VGX_E_ARG;
+    if (n_blocks < 0 || n_blocks > kMaxBlocks) return VGX_E_LIMIT;
+    const int grp = (int)(H / G);
+    if (grp != 1 && grp != 2 && grp != 4 && grp != 6 && grp != 8) return VGX_E_LIMIT;
+    for (int i = 0; i < n_blocks; ++i) {
+        if (blocks[i].n_q < 0 || blocks[i].n_runs < 1 || blocks[i].n_runs > 4) return VGX_E_SIZE;
+        for (int r = 0; r < blocks[i].n_runs; ++r)
+            if (blocks[i].runs[r].len < 0) return VGX_E_SIZE;
+    }
+    return prefill_plan(kKvPair, blocks, n_blocks, G, grp, false).bytes;
+}
+
 int vgx_attn_prefill_ws(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_block *blocks, int n_blocks, int64_t H,
                         int64_t G, int64_t D, float scale, void *workspace, int64_t workspace_bytes, void *stream) {
     if (!workspace) return VGX_E_ARG;
-    return attn_prefill_impl(kv_dtype, q_dtype, out_dtype, blocks, n_blocks, H, G, D, scale, workspace, workspace_bytes,
+    return attn_prefill_impl(kv_dtype, q_dtype, out_dtype, blocks, n_blocks, H, G, D, scale, true, workspace, workspace_bytes,
                              stream);
+}
+
+int vgx_attn_prefill_planes(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_block *blocks, int n_blocks,
+                            int64_t H, int64_t G, int64_t D, float scale, void *workspace, int64_t workspace_bytes,
+                            void *stream) {
+    if (!workspace) return VGX_E_ARG;
+    return attn_prefill_impl(kv_dtype, q_dtype, out_dtype, blocks, n_blocks, H, G, D, scale, false, workspace,
+                             workspace_bytes, stream);
 }
 
 }  // extern "C"

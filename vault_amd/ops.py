@@ -548,8 +548,8 @@ def attn_prefill(blocks, H: int, G: int, scale: Optional[float] = None, ws: Opti
 
     Each block is a dict: ``q`` [n_q, H, D] view (fp32 or bf16, any token / head stride, D contiguous),
     ``out`` [n_q, H, D] view, fp32 or bf16 (one dtype for all blocks), ``runs``: list of (K, V) views
-    [G, n, D] (bf16, or fp32 entering the MFMAs as bf16 hi + lo; one dtype for all runs; D contiguous,
-    any row and group stride), ``causal_base``: -1, or b >= 0 making the last run causal (query t sees
+    [G, n, D] (bf16, or fp32 entering the MFMAs in 16-bit pieces that hold 22 bits or more; one dtype
+    for all runs; D contiguous, any row and group stride), ``causal_base``: -1, or b >= 0 making the last run causal (query t sees
     its keys j <= b + t).  Optional ``bias`` fp32 [n_q, R, >= run length] with ``bias_head_row`` (H
     ints: the bias row of head h, < 0: none) and ``bias_run``: query t of head h adds
     bias[t, bias_head_row[h], j] to its score with key j of that run.  With ``ws`` (a Workspace) a launch
@@ -608,6 +608,13 @@ def attn_prefill(blocks, H: int, G: int, scale: Optional[float] = None, ws: Opti
             buf = ws.get(need)
             L.check(lib.vgx_attn_prefill_ws(KV_DTYPES[kvdt], qd, od, arr, len(part), H, G, D, scale, buf.data_ptr(),
                                             buf.numel(), _stream(part[0]["q"].device)), "vgx_attn_prefill_ws")
+        elif kvdt == torch.float32 and D == 128:
+            # scratch of this call (stream-ordered) for the fp16 planes of K / V
+            need = int(lib.vgx_attn_prefill_planes_bytes(KV_DTYPES[kvdt], arr, len(part), H, G))
+            L.check(min(need, 0), "vgx_attn_prefill_planes_bytes")
+            buf = torch.empty(max(need, 16), dtype=torch.uint8, device=part[0]["q"].device)
+            L.check(lib.vgx_attn_prefill_planes(KV_DTYPES[kvdt], qd, od, arr, len(part), H, G, D, scale, buf.data_ptr(),
+                                                buf.numel(), _stream(part[0]["q"].device)), "vgx_attn_prefill_planes")
         else:
             L.check(lib.vgx_attn_prefill(KV_DTYPES[kvdt], qd, od, arr, len(part), H, G, D, scale,
                                          _stream(part[0]["q"].device)),
