@@ -106,19 +106,32 @@ def block_sliding_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, w
         sinks = sinks.view(B, G, n - 2, S, D)
         # values in the same layout (a K / V run shares one pair of strides)
         sink_v = vb[:, :, :S].reshape(B, G, 1, S, D).expand(B, G, n - 2, S, D).contiguous()
-    blocks = []
+    # the blocks as words: addresses from the strides, no view per block
+    es, ks, ke = kb.element_size(), kb.stride(), kb.data_ptr()
+    ve, qs, os_ = vb.data_ptr(), qq.stride(), out.stride()
+    qe, oe, qp, op = qq.element_size(), out.element_size(), qq.data_ptr(), out.data_ptr()
+    sk, sv = (sinks.data_ptr(), sink_v.data_ptr()) if sinks is not None else (0, 0)
+    none = [0] * 5
+    words = []
     for b in range(B):
+        kb0, vb0 = ke + b * ks[0] * es, ve + b * ks[0] * es
+        qb0, ob0 = qp + b * qs[0] * qe, op + b * os_[0] * oe
         for i in range(n):
             r0, r1 = i * W, min(Lq, (i + 1) * W)
-            runs = []
-            if i >= 2 and S:
-                runs.append((sinks[b, :, i - 2], sink_v[b, :, i - 2]))
+            runs, nr = [], 1
+            if sinks is not None and i >= 2:
+                so = ((b * G) * (n - 2) + i - 2) * S * D * es
+                runs += [sk + so, sv + so, S, D, (n - 2) * S * D]
+                nr += 1
             if i >= 1:
-                runs.append((kb[b, :, r0 - W:r0], vb[b, :, r0 - W:r0]))
-            runs.append((kb[b, :, r0:r1], vb[b, :, r0:r1]))
-            blocks.append({"q": qq[b, :, r0:r1].transpose(0, 1), "out": out[b, :, r0:r1].transpose(0, 1),
-                           "runs": runs, "causal_base": 0})
-    ops.attn_prefill(blocks, H, G)
+                o = (r0 - W) * ks[2] * es
+                runs += [kb0 + o, vb0 + o, W, ks[2], ks[1]]
+                nr += 1
+            o = r0 * ks[2] * es
+            runs += [kb0 + o, vb0 + o, r1 - r0, ks[2], ks[1]]
+            words += [qb0 + r0 * qs[2] * qe, qs[2], qs[1], ob0 + r0 * os_[2] * oe, os_[2], os_[1], r1 - r0, 0, nr]
+            words += runs + none * (4 - nr) + none
+    ops.attn_prefill_words(words, kvdt, qq.dtype, out.dtype, H, G, D, D ** -0.5, q.device)
     return out if out.dtype == q.dtype else out.to(q.dtype)
 
 

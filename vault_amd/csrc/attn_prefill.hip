@@ -1095,7 +1095,8 @@ int64_t vgx_attn_prefill_planes_bytes(int kv_dtype, const vgx_attn_block *blocks
         for (int r = 0; r < blocks[i].n_runs; ++r)
             if (blocks[i].runs[r].len < 0) return VGX_E_SIZE;
     }
-    return prefill_plan(kKvPair, blocks, n_blocks, G, grp, false).bytes;
+    const PrefillPlan p = prefill_plan(kKvPair, blocks, n_blocks, G, grp, false);
+    return p.max_keys >= kPairMinKeys ? p.bytes : 0;
 }
 
 int vgx_attn_prefill_ws(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_block *blocks, int n_blocks, int64_t H,

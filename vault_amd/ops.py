@@ -6,6 +6,7 @@ into the HIP library (no torch fallback).  Tensors must live on a ROCm device.
 from __future__ import annotations
 
 import ctypes as C
+import sys
 from typing import Optional, Tuple
 
 import numpy as np
@@ -602,28 +603,52 @@ def attn_prefill(blocks, H: int, G: int, scale: Optional[float] = None, ws: Opti
                 keep.append((bias, rows_dev))
         qd = L.BF16 if qdt == torch.bfloat16 else L.F32
         od = L.BF16 if odt == torch.bfloat16 else L.F32
-        if ws is not None:
-            need = int(lib.vgx_attn_prefill_workspace_bytes(H, G))
-            L.check(0 if need > 0 else need, "vgx_attn_prefill_workspace_bytes")
-            buf = ws.get(need)
-            L.check(lib.vgx_attn_prefill_ws(KV_DTYPES[kvdt], qd, od, arr, len(part), H, G, D, scale, buf.data_ptr(),
-                                            buf.numel(), _stream(part[0]["q"].device)), "vgx_attn_prefill_ws")
-        elif kvdt == torch.float32 and D == 128:
-            # scratch of this call (stream-ordered) for the fp16 planes of K / V
-            need = int(lib.vgx_attn_prefill_planes_bytes(KV_DTYPES[kvdt], arr, len(part), H, G))
-            L.check(min(need, 0), "vgx_attn_prefill_planes_bytes")
-            buf = torch.empty(max(need, 16), dtype=torch.uint8, device=part[0]["q"].device)
-            L.check(lib.vgx_attn_prefill_planes(KV_DTYPES[kvdt], qd, od, arr, len(part), H, G, D, scale, buf.data_ptr(),
-                                                buf.numel(), _stream(part[0]["q"].device)), "vgx_attn_prefill_planes")
-        else:
-            L.check(lib.vgx_attn_prefill(KV_DTYPES[kvdt], qd, od, arr, len(part), H, G, D, scale,
-                                         _stream(part[0]["q"].device)),
-                    "vgx_attn_prefill")
+        _prefill_launch(C.addressof(arr), len(part), kvdt, qd, od, H, G, D, scale, ws, part[0]["q"].device)
 
 
-# ------------------------------------------------------------------------------------------
-# segment bank and token selection
-# ------------------------------------------------------------------------------------------
+# vgx_attn_block as 64-bit words (its two ints are padded to 8 bytes): q, ldq, q_hstride, out, ldo, o_hstride, n_q,
+# causal_base, n_runs, four runs of (k, v, len, row_stride, group_stride), bias, bias_head_row, bias_ldq,
+# bias_rstride, bias_run
+PREFILL_BLOCK_WORDS = 34
+assert C.sizeof(L.AttnBlock) == 8 * PREFILL_BLOCK_WORDS and sys.byteorder == "little"
+
+
+def attn_prefill_words(words: list, kvdt: torch.dtype, qdt: torch.dtype, odt: torch.dtype, H: int, G: int,
+                       D: int, scale: float, dev: torch.device) -> None:
+    """attn_prefill over blocks given as PREFILL_BLOCK_WORDS words each, for callers whose blocks are
+    regular: filling them from tensor views costs the host about 20 us a block, a list of words 3."""
+    arr = (C.c_int64 * len(words))(*words)
+    n = len(words) // PREFILL_BLOCK_WORDS
+    qd = L.BF16 if qdt == torch.bfloat16 else L.F32
+    od = L.BF16 if odt == torch.bfloat16 else L.F32
+    for i0 in range(0, n, 8):
+        _prefill_launch(C.addressof(arr) + 8 * PREFILL_BLOCK_WORDS * i0, min(8, n - i0), kvdt, qd, od, H, G, D, scale,
+                        None, dev)
+
+
+def _prefill_launch(blocks: int, n: int, kvdt: torch.dtype, qd: int, od: int, H: int, G: int, D: int, scale: float,
+                    ws: Optional["Workspace"], dev: torch.device) -> None:
+    lib = L.load()
+    kd = KV_DTYPES[kvdt]
+    need = 0
+    if ws is not None:
+        need = int(lib.vgx_attn_prefill_workspace_bytes(H, G))
+        L.check(0 if need > 0 else need, "vgx_attn_prefill_workspace_bytes")
+        buf = ws.get(need)
+        L.check(lib.vgx_attn_prefill_ws(kd, qd, od, blocks, n, H, G, D, scale, buf.data_ptr(), buf.numel(), _stream(dev)),
+                "vgx_attn_prefill_ws")
+        return
+    if kvdt == torch.float32 and D == 128:
+        need = int(lib.vgx_attn_prefill_planes_bytes(kd, blocks, n, H, G))
+        L.check(min(need, 0), "vgx_attn_prefill_planes_bytes")
+    if need:
+        # scratch of this call (stream-ordered) for the fp16 planes of K / V
+        buf = torch.empty(need, dtype=torch.uint8, device=dev)
+        L.check(lib.vgx_attn_prefill_planes(kd, qd, od, blocks, n, H, G, D, scale, buf.data_ptr(), need, _stream(dev)),
+                "vgx_attn_prefill_planes")
+    else:
+        L.check(lib.vgx_attn_prefill(kd, qd, od, blocks, n, H, G, D, scale, _stream(dev)), "vgx_attn_prefill")
+
 
 def seg_step(ids: torch.Tensor, step: torch.Tensor, tok_cur: torch.Tensor, seg_cur: Optional[torch.Tensor],
              ctrl: Optional[torch.Tensor], tiers: Optional[torch.Tensor], seg_min: int, seg_max: int) -> None:
