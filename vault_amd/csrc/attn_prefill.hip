@@ -33,8 +33,8 @@
 // each) and probabilities are split the same way, and each product keeps hi x hi, hi x lo and lo x hi.  The K scale
 // multiplies the scores; the V scale enters the weights' exponent, so it is part of the running max, and is taken out
 // of the sum.  Three MFMAs per product and no conversions in the tile loop instead of six and the staging below:
-// two sequences of 2500 at 12 / 2 heads 359 -> 186 us, at 4 / 4 heads 887 -> 174 (what is left there is the host's
-// side of the call); relative error against 64 bits 4.4e-7 -> 3.5e-7.  At 3584 keys the kernel takes 76 us for 1024
+// two sequences of 2500 at 12 / 2 heads 348 -> 178 us, at 4 / 4 heads 885 -> 170 (the whole call);
+// relative error against 64 bits 4.4e-7 -> 3.5e-7.  At 3584 keys the kernel takes 76 us for 1024
 // queries (19.3 GFLOP, its MFMAs 23 us at peak): the chain scores -> softmax -> P V of three waves per SIMD and
 // 32 KB of LDS reads per wave and 32 keys bound it.
 // Without that workspace, for few keys, or with key ranges (vgx_attn_prefill_ws), each fp32 tile is loaded into registers during the previous tile's
