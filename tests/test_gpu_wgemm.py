@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from oracle import codec, linalg
+from vault_amd import _lib as L
 from vault_amd import ops, vlt3
 
 pytestmark = pytest.mark.gpu
@@ -60,3 +61,23 @@ def test_wgemm_matches_oracle(dev, dt, rows, cols, batch, epi):
     if epi == "edge":
         nz = wf[:, 7] != 0
         assert np.all(np.isinf(y[4][nz])) and np.all(np.isnan(y[4][~nz])) and np.all(np.isnan(y[5]))
+
+
+@pytest.mark.parametrize("dt", [codec.BF16, codec.F16])
+def test_wgemm_leaves_the_tile_counters(dev, dt):
+    """One zero-filled workspace for a 16-bit GEMM and then a Q4_0 decode batch whose workgroups take tickets from
+    its counters (the down projection of a batch of 16)."""
+    lib, rng = L.load(), np.random.default_rng(3)
+    B, d, ff = 16, 1536, 8960
+    raw = vlt3.synthetic_blocks(codec.Q4_0, d, ff, rng)
+    w4, wf = ops.QWeight.from_blocks(codec.Q4_0, d, ff, raw, dev), codec.decode(codec.Q4_0, raw, d, ff)
+    wb = ops.QWeight.from_blocks(dt, d, ff, vlt3.quantize(dt, np.ones((d, ff), np.float32)), dev)
+    x = rng.standard_normal((B, ff)).astype(np.float32)
+    xt, y = torch.from_numpy(x).to(dev), torch.full((B, d), 7.0, device=dev)
+    ws = torch.zeros(int(lib.vgx_qgemm_workspace_bytes(B, d, ff, L.EPI_STORE)), dtype=torch.uint8, device=dev)
+    for w in (wb, w4):
+        L.check(lib.vgx_qgemm(w.dtype, w.packed.data_ptr(), d, ff, xt.data_ptr(), ff, B, None, 0.0, None, y.data_ptr(), d,
+                              L.EPI_STORE, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream), "vgx_qgemm")
+    assert int(ws[:65536].max()) == 0
+    err = np.abs(y.cpu().numpy() - linalg.gemv(wf, x))
+    assert np.all(err <= linalg.gemv_bound(wf, x, codec.Q4_0))

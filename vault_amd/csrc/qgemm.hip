@@ -2424,7 +2424,8 @@ int split_proj_launch(int dtype, const void *wp, int64_t rows, int64_t cols, con
     return ks;
 }
 
-// BF16 / F16 weights on wgemm_tile_kernel: planes, per-row scales, K-split partials.
+// BF16 / F16 weights on wgemm_tile_kernel: planes, per-row scales, K-split partials, past the tile counters
+// (which the next decode batch on the same workspace takes its tickets from).
 constexpr int kWgTM = 256, kWgTN = 64, kWgNS = 2;
 // K splits: as many as fit 512 workgroups (one round at two per CU), at least 8 blocks each.
 inline int wgemm_ksplit(int64_t n_rq, int64_t batch, int nblk) {
@@ -2435,7 +2436,7 @@ inline int wgemm_ksplit(int64_t n_rq, int64_t batch, int nblk) {
 }
 inline int64_t wgemm_bytes(int64_t batch, int64_t n_rq, int nblk) {
     const int64_t cols = (int64_t)nblk * QK;
-    return 3 * split_plane_bytes(batch, cols) + (batch * 4 + 255) / 256 * 256 +
+    return kQgemmTicketBytes + 3 * split_plane_bytes(batch, cols) + (batch * 4 + 255) / 256 * 256 +
            part_bytes(wgemm_ksplit(n_rq, batch, nblk), batch, n_rq * 4);
 }
 
@@ -2444,7 +2445,7 @@ int wgemm_launch(const void *w_packed, int64_t rows, int64_t n_rq, int nblk, con
                  const float *bias, float *y, int64_t ldy, int epilogue, void *workspace, hipStream_t st) {
     const int cols = nblk * QK;
     const int64_t pb = split_plane_bytes(batch, cols);
-    char *const ws = static_cast<char *>(workspace);
+    char *const ws = static_cast<char *>(workspace) + kQgemmTicketBytes;
     auto *xs = reinterpret_cast<uint16_t *>(ws);
     float *xsc = nullptr;
     if constexpr (WDT == VGX_BF16) {
