@@ -81,3 +81,42 @@ def test_wgemm_leaves_the_tile_counters(dev, dt):
     assert int(ws[:65536].max()) == 0
     err = np.abs(y.cpu().numpy() - linalg.gemv(wf, x))
     assert np.all(err <= linalg.gemv_bound(wf, x, codec.Q4_0))
+
+
+@pytest.mark.parametrize("dt", [codec.BF16, codec.F16])
+@pytest.mark.parametrize("rows,cols,batch", [(70, 96, 9), (258, 1536, 70)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_wgemm_infinities(dev, dt, rows, cols, batch, swiglu):
+    """Infinite and NaN weights and activations (one K range and several): against activations of few bits, whose lower
+    pieces are zero, against zeros, each other and ordinary elements.  An output is infinite or NaN where the float64
+    product is, and within the usual bound elsewhere."""
+    rng = np.random.default_rng(rows)
+    td = torch.bfloat16 if dt == codec.BF16 else torch.float16
+
+    def mk():
+        w = (rng.standard_normal((rows, cols)) * 0.05).astype(np.float32)
+        w[3, 7], w[4, 7], w[5, 9], w[6, 7], w[6, 8], w[rows - 1, cols - 1] = np.inf, -np.inf, np.nan, np.inf, -np.inf, np.inf
+        w[7:9, 7], w[9, 11] = 0.5, 0.0
+        return torch.from_numpy(w).to(td)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    x[1, 7], x[2, 7], x[3, 7], x[4, 11], x[5, 3], x[6, 8] = 1.0, np.inf, 0.0, -np.inf, np.nan, -np.inf
+    x[batch - 1, cols - 1] = -2.0
+    blocks = lambda t: t.view(torch.uint8).reshape(-1)  # noqa: E731
+    ws = [mk() for _ in range(2 if swiglu else 1)]
+    xd = torch.from_numpy(x).to(dev)
+    if swiglu:
+        y = ops.qlinear_swiglu(ops.QWeight.gateup_from_blocks(dt, rows, cols, blocks(ws[0]), blocks(ws[1]), dev), xd)
+    else:
+        y = ops.qlinear(ops.QWeight.from_blocks(dt, rows, cols, blocks(ws[0]), dev), xd)
+    y = y.double().cpu().numpy()
+    wf = [w.double().numpy() for w in ws]
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = [np.stack([(w * xb.astype(np.float64)).sum(1) for xb in x]) for w in wf]
+        out = linalg.swiglu(*ref) if swiglu else ref[0]
+    inf, fin = np.isinf(out), np.isfinite(out)
+    assert np.array_equal(np.isnan(y), np.isnan(out)) and np.array_equal(y[inf], out[inf])
+    bound = [linalg.gemv_bound(np.nan_to_num(w, nan=0.0, posinf=0.0, neginf=0.0).astype(np.float32),
+                               np.nan_to_num(x, nan=0.0, posinf=0.0, neginf=0.0), dt) for w in wf]
+    with np.errstate(invalid="ignore"):
+        tol = 1.1 * np.abs(ref[1]) * bound[0] + np.abs(ref[0]) * bound[1] + 1e-6 * np.abs(out) if swiglu else bound[0]
+    assert np.all(np.abs(y[fin] - out[fin]) <= tol[fin] + 1e-30)

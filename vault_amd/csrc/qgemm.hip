@@ -2462,7 +2462,9 @@ int wgemm_launch(const void *w_packed, int64_t rows, int64_t n_rq, int nblk, con
     const int ks = wgemm_ksplit(n_rq, batch, nblk), kper = (nblk + ks - 1) / ks;
     const dim3 grid((unsigned)((n_rq + kWgTM / 4 - 1) / (kWgTM / 4)), (unsigned)((batch + kWgTN - 1) / kWgTN), (unsigned)ks);
     const auto *w = static_cast<const uint8_t *>(w_packed);
-#define VGX_WG(EPI, SP)                                                                                            hipLaunchKernelGGL((wgemm_tile_kernel<WDT, EPI, SP, kWgTM, kWgTN, kWgNS>), grid, dim3(kWgTM * kWgTN / 64), 0, st, w,                        n_rq, nblk, rows, xs, pb / 2, xsc, batch, bias, y, ldy, part, kper)
+#define VGX_WG(EPI, SP)                                                                                            \
+    hipLaunchKernelGGL((wgemm_tile_kernel<WDT, EPI, SP, kWgTM, kWgTN, kWgNS>), grid, dim3(kWgTM * kWgTN / 64), 0, st, w, \
+                       n_rq, nblk, rows, xs, pb / 2, xsc, x, ldx, batch, bias, y, ldy, part, kper)
     if (ks > 1) VGX_WG(EPI_STORE, true);
     else if (epilogue == VGX_EPI_SWIGLU) VGX_WG(EPI_SWIGLU, false);
     else if (epilogue == VGX_EPI_ACCUM) VGX_WG(EPI_ACCUM, false);

@@ -22,8 +22,7 @@ template <int WDT>
 constexpr int kPlanes = WDT == VGX_BF16 ? 3 : 2;
 
 // Three bf16 planes of the activations, natural order: plane p of row b at xs + p * pstride + b * cols.
-// A non-finite element keeps its bf16 value in the first plane and zeros in the others, so that an
-// infinity reaches the outputs as an infinity.  One thread per four elements.
+// One thread per four elements.
 __global__ __launch_bounds__(256) void xsplit_bf16x3_kernel(const float *__restrict__ x, int64_t ldx, int cols,
                                                              int64_t n4, uint16_t *__restrict__ xs, int64_t pstride) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -42,14 +41,10 @@ __global__ __launch_bounds__(256) void xsplit_bf16x3_kernel(const float *__restr
     uint32_t h[4], m[4], l[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const bool fin = __builtin_isfinite(e[k]);
-        const uint32_t hb = __float_as_uint(e[k]) & 0xFFFF0000u;
-        const float r = e[k] - __uint_as_float(hb);                 // exact: the low 16 mantissa bits
-        const uint32_t mb = __float_as_uint(r) & 0xFFFF0000u;
-        const float q = r - __uint_as_float(mb);                    // exact: at most 8 bits
-        h[k] = fin ? hb : float_to_bf16_bits(e[k]) << 16;
-        m[k] = fin ? mb : 0u;
-        l[k] = fin ? __float_as_uint(q) : 0u;
+        h[k] = __float_as_uint(e[k]) & 0xFFFF0000u;
+        const float r = e[k] - __uint_as_float(h[k]);               // exact: the low 16 mantissa bits
+        m[k] = __float_as_uint(r) & 0xFFFF0000u;
+        l[k] = __float_as_uint(r - __uint_as_float(m[k]));          // exact: at most 8 bits
     }
     const auto put = [&](int p, const uint32_t (&v)[4]) {
         *reinterpret_cast<uint2 *>(xs + p * pstride + b * cols + c) =
@@ -58,6 +53,24 @@ __global__ __launch_bounds__(256) void xsplit_bf16x3_kernel(const float *__restr
     put(0, h);
     put(1, m);
     put(2, l);
+}
+
+// One output of blocks blk_lo .. blk_hi - 1 from the operands as they are, for the outputs that the pieces make
+// NaN: an infinite weight or activation meets a piece that is zero (or the rest of an infinity), where the product
+// itself is an infinity or NaN as the other factor says.
+template <int WDT>
+__device__ float wgemm_plain_dot(const uint8_t *__restrict__ W, int nblk, int64_t row, int blk_lo, int blk_hi,
+                                 const float *__restrict__ xr) {
+    const uint16_t *wr = reinterpret_cast<const uint16_t *>(W) + ((row >> 2) * nblk * 4 + (row & 3)) * QK;
+    float s = 0.0f;
+#pragma unroll 1
+    for (int blk = blk_lo; blk < blk_hi; ++blk)
+#pragma unroll 4
+        for (int j = 0; j < QK; ++j) {
+            const uint32_t w = wr[(int64_t)blk * 4 * QK + j];
+            s = fmaf(WDT == VGX_BF16 ? bf16_bits_to_float(w) : half_bits_to_float(w), xr[blk * QK + j], s);
+        }
+    return s;
 }
 
 // Tile of TM weight rows x TN activation rows, a wave 64 x 64 (wave w: weight rows 64 (w % (TM / 64)),
@@ -73,8 +86,8 @@ __global__ __launch_bounds__(256) void xsplit_bf16x3_kernel(const float *__restr
 template <int WDT, int EPI, bool SPLIT, int TM, int TN, int NS>
 __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm_tile_kernel(
     const uint8_t *__restrict__ W, int64_t n_rq, int nblk, int64_t rows_out, const uint16_t *__restrict__ xs,
-    int64_t pstride, const float *__restrict__ xscale, int64_t batch, const float *__restrict__ bias,
-    float *__restrict__ y, int64_t ldy, float *__restrict__ part, int kper) {
+    int64_t pstride, const float *__restrict__ xscale, const float *__restrict__ x, int64_t ldx, int64_t batch,
+    const float *__restrict__ bias, float *__restrict__ y, int64_t ldy, float *__restrict__ part, int kper) {
     constexpr int NP = kPlanes<WDT>;
     constexpr int NWAVE = TM / 64 * (TN / 64);
     constexpr int NT = 64 * NWAVE;
@@ -182,6 +195,7 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the stages are free for the epilogue
 
     if constexpr (SPLIT) {
+        bool bad = false;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const int64_t b = b0 + wn * 64 + 16 * c + l16;
@@ -194,6 +208,16 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
                 float4 v;
                 v.x = acc[t][c][0] * sc; v.y = acc[t][c][1] * sc; v.z = acc[t][c][2] * sc; v.w = acc[t][c][3] * sc;
                 *reinterpret_cast<float4 *>(part + ((int64_t)blockIdx.z * batch + b) * (n_rq * 4) + crq * 4) = v;
+                bad |= !(v.x == v.x && v.y == v.y && v.z == v.z && v.w == v.w);
+            }
+        }
+        if (bad) {
+#pragma unroll 1
+            for (int e = 0; e < 64; ++e) {
+                const int64_t b = b0 + wn * 64 + 16 * (e >> 4) + l16, crq = rq0 + wm * 16 + (e >> 2 & 3) * 4 + lg;
+                if (b >= batch || crq >= n_rq) continue;
+                float *pe = part + ((int64_t)blockIdx.z * batch + b) * (n_rq * 4) + crq * 4 + (e & 3);
+                if (__builtin_isnan(*pe)) *pe = wgemm_plain_dot<WDT>(W, nblk, crq * 4 + (e & 3), blk_lo, blk_hi, x + b * ldx);
             }
         }
         return;
@@ -223,7 +247,10 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
                 if (b >= batch || oo >= rows_out) continue;
                 const float *er = et + bl_ * kERow + (o >> 1) * 4 + (o & 1);
                 const float sc = et[bl_ * kERow + 64];
-                const float g = er[0] * sc, u = er[2] * sc;
+                float g = er[0] * sc, u = er[2] * sc;
+                const int64_t row = r0 + (o >> 1) * 4 + (o & 1);
+                if (__builtin_isnan(g)) g = wgemm_plain_dot<WDT>(W, nblk, row, 0, nblk, x + b * ldx);
+                if (__builtin_isnan(u)) u = wgemm_plain_dot<WDT>(W, nblk, row + 2, 0, nblk, x + b * ldx);
                 y[b * ldy + oo] = g / (1.0f + __expf(-g)) * u;
             }
         } else {
@@ -232,6 +259,7 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
                 const int64_t b = b0 + bl_, row = r0 + rr;
                 if (b >= batch || row >= rows_out) continue;
                 float v = et[bl_ * kERow + rr] * et[bl_ * kERow + 64];
+                if (__builtin_isnan(v)) v = wgemm_plain_dot<WDT>(W, nblk, row, 0, nblk, x + b * ldx);
                 if (bias) v += bias[row];
                 if constexpr (EPI == EPI_ACCUM) v += y[b * ldy + row];
                 y[b * ldy + row] = v;
