@@ -1,8 +1,8 @@
 """GPU parity of the BF16 / F16 GEMM on the 16-bit matrix cores (vgx_qgemm with a workspace, used by
 ops.qlinear from 8 activation rows on) against the fp64 oracle.
 
-Bar: the fp32 accumulation bound at the one-row GEMV's relative term (2e-6).  The pieces hold 24 (BF16)
-and about 22 (F16) bits of the activations, 2^-22 at most, a tenth of it."""
+Bar: the fp32 accumulation bound at the one-row GEMV's relative term (2e-6).  The pieces hold the whole
+significand of every activation under its own exponent."""
 import numpy as np
 import pytest
 import torch
@@ -120,3 +120,20 @@ def test_wgemm_infinities(dev, dt, rows, cols, batch, swiglu):
     with np.errstate(invalid="ignore"):
         tol = 1.1 * np.abs(ref[1]) * bound[0] + np.abs(ref[0]) * bound[1] + 1e-6 * np.abs(out) if swiglu else bound[0]
     assert np.all(np.abs(y[fin] - out[fin]) <= tol[fin] + 1e-30)
+
+
+@pytest.mark.parametrize("dt", [codec.BF16, codec.F16])
+@pytest.mark.parametrize("big", [1e4, 1e10, 1e30])
+def test_wgemm_elements_keep_their_own_exponent(dev, dt, big):
+    """A large activation that meets zero weights costs the rest of its row nothing (the bound counts only what the
+    weights multiply), whether it stands in one row or in all."""
+    rng = np.random.default_rng(1)
+    rows, cols, batch = 70, 544, 40
+    w = (rng.standard_normal((rows, cols)) * 0.05).astype(np.float32)
+    w[:, 5] = 0.0
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    x[::2, 5] = big
+    raw = vlt3.quantize(dt, w)
+    wf = codec.decode(dt, raw, rows, cols)
+    y = ops.qlinear(ops.QWeight.from_blocks(dt, rows, cols, raw, dev), torch.from_numpy(x).to(dev)).cpu().numpy()
+    assert np.all(np.abs(y - linalg.gemv(wf, x)) <= linalg.gemv_bound(wf, x, dt))

@@ -52,12 +52,9 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // so 2^-k is a normal float; a row holding an infinity or a NaN is not scaled (k = 0), so that it
 // reaches the outputs as it would unsplit.
 // Inside every group of four, elements 1 and 2 trade places (stored order 0, 2, 1, 3): the K-slot
-// order of the tiled kernel's weight fragments, whose Q4_0 nibble pairs come out of a word that way;
-// with NATURAL (F16 weights, wgemm_tile_kernel) they stay in place, and a non-finite element gets a zero
-// lo, so that an infinity reaches the outputs as one.
+// order of the tiled kernel's weight fragments, whose Q4_0 nibble pairs come out of a word that way.
 // One workgroup of 256 threads per activation row.
 constexpr int kXsplitRegs = 20;   // float4 per thread kept in registers: rows of up to 20480 elements
-template <bool NATURAL = false>
 __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x, int64_t ldx,
                                                       const float *__restrict__ lnw, float eps, int cols,
                                                       uint16_t *__restrict__ xh, uint16_t *__restrict__ xl,
@@ -129,15 +126,6 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x
             v.x = g.x * (v.x * inv); v.y = g.y * (v.y * inv); v.z = g.z * (v.z * inv); v.w = g.w * (v.w * inv);
         }
         v.x *= sc; v.y *= sc; v.z *= sc; v.w *= sc;
-        if constexpr (NATURAL) {
-            const uint32_t h01 = pack_f16x2(v.x, v.y), h23 = pack_f16x2(v.z, v.w);
-            const auto hp = __builtin_bit_cast(vgx_f16x2_t, h01), hq = __builtin_bit_cast(vgx_f16x2_t, h23);
-            auto rest = [](float e, _Float16 h) { return __builtin_isfinite(e) ? e - (float)h : 0.0f; };
-            *reinterpret_cast<uint2 *>(xh + b * cols + 4 * i) = make_uint2(h01, h23);
-            *reinterpret_cast<uint2 *>(xl + b * cols + 4 * i) =
-                make_uint2(pack_f16x2(rest(v.x, hp[0]), rest(v.y, hp[1])), pack_f16x2(rest(v.z, hq[0]), rest(v.w, hq[1])));
-            return;
-        }
         // stored order 0, 2, 1, 3
         const uint32_t h02 = pack_f16x2(v.x, v.z), h13 = pack_f16x2(v.y, v.w);
         const auto hp = __builtin_bit_cast(vgx_f16x2_t, h02), hq = __builtin_bit_cast(vgx_f16x2_t, h13);
@@ -2424,7 +2412,7 @@ int split_proj_launch(int dtype, const void *wp, int64_t rows, int64_t cols, con
     return ks;
 }
 
-// BF16 / F16 weights on wgemm_tile_kernel: planes, per-row scales, K-split partials, past the tile counters
+// BF16 / F16 weights on wgemm_tile_kernel: planes, K-split partials, past the tile counters
 // (which the next decode batch on the same workspace takes its tickets from).
 constexpr int kWgTM = 256, kWgTN = 64, kWgNS = 2;
 // K splits: as many as fit 512 workgroups (one round at two per CU), at least 8 blocks each.
@@ -2436,7 +2424,7 @@ inline int wgemm_ksplit(int64_t n_rq, int64_t batch, int nblk) {
 }
 inline int64_t wgemm_bytes(int64_t batch, int64_t n_rq, int nblk) {
     const int64_t cols = (int64_t)nblk * QK;
-    return kQgemmTicketBytes + 3 * split_plane_bytes(batch, cols) + (batch * 4 + 255) / 256 * 256 +
+    return kQgemmTicketBytes + kPlanes * split_plane_bytes(batch, cols) +
            part_bytes(wgemm_ksplit(n_rq, batch, nblk), batch, n_rq * 4);
 }
 
@@ -2447,24 +2435,16 @@ int wgemm_launch(const void *w_packed, int64_t rows, int64_t n_rq, int nblk, con
     const int64_t pb = split_plane_bytes(batch, cols);
     char *const ws = static_cast<char *>(workspace) + kQgemmTicketBytes;
     auto *xs = reinterpret_cast<uint16_t *>(ws);
-    float *xsc = nullptr;
-    if constexpr (WDT == VGX_BF16) {
-        const int64_t n4 = batch * (cols / 4);
-        hipLaunchKernelGGL(xsplit_bf16x3_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, x, ldx, cols, n4, xs,
-                           pb / 2);
-    } else {
-        xsc = reinterpret_cast<float *>(ws + 3 * pb);
-        hipLaunchKernelGGL(xsplit_kernel<true>, dim3((unsigned)batch), dim3(256), 0, st, x, ldx, nullptr, 0.0f, cols, xs,
-                           xs + pb / 2, xsc);
-    }
+    const int64_t n4 = batch * (cols / 4);
+    hipLaunchKernelGGL(xsplit_bf16x3_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, x, ldx, cols, n4, xs, pb / 2);
     VGX_CHECK_LAUNCH();
-    auto *part = reinterpret_cast<float *>(ws + 3 * pb + (batch * 4 + 255) / 256 * 256);
+    auto *part = reinterpret_cast<float *>(ws + kPlanes * pb);
     const int ks = wgemm_ksplit(n_rq, batch, nblk), kper = (nblk + ks - 1) / ks;
     const dim3 grid((unsigned)((n_rq + kWgTM / 4 - 1) / (kWgTM / 4)), (unsigned)((batch + kWgTN - 1) / kWgTN), (unsigned)ks);
     const auto *w = static_cast<const uint8_t *>(w_packed);
 #define VGX_WG(EPI, SP)                                                                                            \
     hipLaunchKernelGGL((wgemm_tile_kernel<WDT, EPI, SP, kWgTM, kWgTN, kWgNS>), grid, dim3(kWgTM * kWgTN / 64), 0, st, w, \
-                       n_rq, nblk, rows, xs, pb / 2, xsc, x, ldx, batch, bias, y, ldy, part, kper)
+                       n_rq, nblk, rows, xs, pb / 2, x, ldx, batch, bias, y, ldy, part, kper)
     if (ks > 1) VGX_WG(EPI_STORE, true);
     else if (epilogue == VGX_EPI_SWIGLU) VGX_WG(EPI_SWIGLU, false);
     else if (epilogue == VGX_EPI_ACCUM) VGX_WG(EPI_ACCUM, false);
@@ -2523,7 +2503,7 @@ int vgx_qgemm(int dtype, const void *w_packed, int64_t rows, int64_t cols, const
         // fit the DMA's buffer ranges; without one (it is optional here) on the fp32 MFMA.  Gate/up | down
         // of BF16 files at 8, 40, 333, 1024 rows: 107 -> 25, 108 -> 33, 243 -> 76, 591 -> 184 us | 472 ->
         // 24, 474 -> 28, 462 -> 53, 467 -> 107 us: ahead at every batch size this entry takes
-        const int64_t pbytes = 3 * split_plane_bytes(batch, cols);
+        const int64_t pbytes = kPlanes * split_plane_bytes(batch, cols);
         if (dtype != VGX_F32 && workspace && (uintptr_t)workspace % 256 == 0 &&
             workspace_bytes >= wgemm_bytes(batch, n_rq, nblk) && n_rq * nblk * 256 < ((int64_t)1 << 31) &&
             pbytes < ((int64_t)1 << 31)) {
@@ -2667,7 +2647,7 @@ int vgx_qgemm(int dtype, const void *w_packed, int64_t rows, int64_t cols, const
     auto *xl = reinterpret_cast<uint16_t *>(wsb + pb);
     auto *xsc = reinterpret_cast<float *>(wsb + 2 * pb);
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(xsplit_kernel<false>, dim3((unsigned)batch), dim3(256), 0, st, x, ldx, norm_w, eps, (int)cols, xh, xl,
+    hipLaunchKernelGGL(xsplit_kernel, dim3((unsigned)batch), dim3(256), 0, st, x, ldx, norm_w, eps, (int)cols, xh, xl,
                        xsc);
     VGX_CHECK_LAUNCH();
     auto *part = reinterpret_cast<float *>(wsb + split_bytes(batch, cols));

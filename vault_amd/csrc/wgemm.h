@@ -3,11 +3,11 @@
 //
 // Reference semantics: the F32-accumulated product of runtime/vault3.c:499-535 over a block of rows.
 //
-// Exactness.  The weights enter the MFMA as they are.  BF16 weights: the activations as three bf16
-// pieces cut from the fp32 mantissa by truncation (8 + 8 + 8 bits: every product is exact and the pieces
-// add up to the activation, but for pieces below bf16's normal range).  F16 weights: fp16 hi + lo of the
-// row scaled by a power of two (xsplit_kernel, about 22 bits).  All pieces of a block accumulate into one
-// fp32 accumulator.
+// Exactness.  The activations enter as three bf16 pieces cut from the fp32 mantissa by truncation (8 + 8 + 8
+// bits, each element under its own exponent: every product is exact and the pieces add up to the activation,
+// but for pieces below bf16's normal range).  BF16 weights enter as they are, F16 weights as two bf16 pieces
+// (8 + 3 bits, exact over fp16's whole range), widened from the staged tile.  All pieces of a block accumulate
+// into one fp32 accumulator.
 //
 // What bounds it: at chunk sizes the matrix cores at three (two) times the product's operations (gate/up
 // 2 x 8960 x 1536 over 1024 rows: 184 us, 306 TFLOP/s of the product, 920 of the pieces, against 1200 of
@@ -18,8 +18,7 @@
 
 namespace {
 
-template <int WDT>
-constexpr int kPlanes = WDT == VGX_BF16 ? 3 : 2;
+constexpr int kPlanes = 3;
 
 // Three bf16 planes of the activations, natural order: plane p of row b at xs + p * pstride + b * cols.
 // One thread per four elements.
@@ -55,6 +54,21 @@ __global__ __launch_bounds__(256) void xsplit_bf16x3_kernel(const float *__restr
     put(2, l);
 }
 
+// Eight fp16 weights as bf16 pieces: hi the leading 8 bits of the significand, lo the other 3.
+__device__ __forceinline__ void widen_f16x8(uint4 h, uint4 &hi, uint4 &lo) {
+    const uint32_t w[4] = {h.x, h.y, h.z, h.w};
+    uint32_t hv[4], lv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = half_bits_to_float(w[i]), b = half_bits_to_float(w[i] >> 16);
+        const uint32_t ha = __float_as_uint(a) & 0xFFFF0000u, hb = __float_as_uint(b) & 0xFFFF0000u;
+        hv[i] = ha >> 16 | hb;
+        lv[i] = __float_as_uint(a - __uint_as_float(ha)) >> 16 | (__float_as_uint(b - __uint_as_float(hb)) & 0xFFFF0000u);
+    }
+    hi = make_uint4(hv[0], hv[1], hv[2], hv[3]);
+    lo = make_uint4(lv[0], lv[1], lv[2], lv[3]);
+}
+
 // One output of blocks blk_lo .. blk_hi - 1 from the operands as they are, for the outputs that the pieces make
 // NaN: an infinite weight or activation meets a piece that is zero (or the rest of an infinity), where the product
 // itself is an infinity or NaN as the other factor says.
@@ -86,9 +100,10 @@ __device__ float wgemm_plain_dot(const uint8_t *__restrict__ W, int nblk, int64_
 template <int WDT, int EPI, bool SPLIT, int TM, int TN, int NS>
 __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm_tile_kernel(
     const uint8_t *__restrict__ W, int64_t n_rq, int nblk, int64_t rows_out, const uint16_t *__restrict__ xs,
-    int64_t pstride, const float *__restrict__ xscale, const float *__restrict__ x, int64_t ldx, int64_t batch,
-    const float *__restrict__ bias, float *__restrict__ y, int64_t ldy, float *__restrict__ part, int kper) {
-    constexpr int NP = kPlanes<WDT>;
+    int64_t pstride, const float *__restrict__ x, int64_t ldx, int64_t batch, const float *__restrict__ bias,
+    float *__restrict__ y, int64_t ldy, float *__restrict__ part, int kper) {
+    constexpr int NP = kPlanes;
+    constexpr int NW = WDT == VGX_F16 ? 2 : 1;         // bf16 pieces of a weight
     constexpr int NWAVE = TM / 64 * (TN / 64);
     constexpr int NT = 64 * NWAVE;
     constexpr int A_B = TM * QK * 2, BH_B = TN * QK * 2;
@@ -157,25 +172,24 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
     };
     auto compute = [&](int buf) {
         const int s0 = buf * STAGE_B;
-        uint4 af[4];
+        uint4 af[NW][4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) af[t] = frag(s0, wm * 64 + 16 * t + l16);
+        for (int t = 0; t < 4; ++t) {
+            af[0][t] = frag(s0, wm * 64 + 16 * t + l16);
+            if constexpr (WDT == VGX_F16) widen_f16x8(af[0][t], af[0][t], af[NW - 1][t]);
+        }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
                 const uint4 bf = frag(s0 + A_B + p * BH_B, wn * 64 + 16 * c + l16);
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    if constexpr (WDT == VGX_BF16)
-                        acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, af[t]),
+                for (int w = 0; w < NW; ++w)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, af[w][t]),
                                                                              __builtin_bit_cast(bf16x8_t, bf), acc[t][c],
                                                                              0, 0, 0);
-                    else
-                        acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, af[t]),
-                                                                            __builtin_bit_cast(f16x8_t, bf), acc[t][c],
-                                                                            0, 0, 0);
-                }
             }
         }
     };
@@ -194,48 +208,59 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the stages are free for the epilogue
 
+    auto any_nan = [](float4 v) { return !(v.x == v.x && v.y == v.y && v.z == v.z && v.w == v.w); };
+    // this lane's NaN sums, four rows at at(t, b, crq, c), computed again
+    auto repair = [&](auto at) {
+#pragma unroll 1
+        for (int e = 0; e < 16; ++e) {
+            const int c = e >> 2, t = e & 3;
+            const int64_t b = b0 + wn * 64 + 16 * c + l16, crq = rq0 + wm * 16 + 4 * t + lg;
+            if (b >= batch || crq >= n_rq) continue;
+            float *v = at(t, b, crq, c);
+#pragma unroll 1
+            for (int i = 0; i < 4; ++i)
+                if (__builtin_isnan(v[i])) v[i] = wgemm_plain_dot<WDT>(W, nblk, crq * 4 + i, blk_lo, blk_hi, x + b * ldx);
+        }
+    };
     if constexpr (SPLIT) {
         bool bad = false;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const int64_t b = b0 + wn * 64 + 16 * c + l16;
             if (b >= batch) continue;
-            const float sc = xscale ? xscale[b] : 1.0f;
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const int64_t crq = rq0 + wm * 16 + 4 * t + lg;
                 if (crq >= n_rq) continue;
                 float4 v;
-                v.x = acc[t][c][0] * sc; v.y = acc[t][c][1] * sc; v.z = acc[t][c][2] * sc; v.w = acc[t][c][3] * sc;
+                v.x = acc[t][c][0]; v.y = acc[t][c][1]; v.z = acc[t][c][2]; v.w = acc[t][c][3];
                 *reinterpret_cast<float4 *>(part + ((int64_t)blockIdx.z * batch + b) * (n_rq * 4) + crq * 4) = v;
-                bad |= !(v.x == v.x && v.y == v.y && v.z == v.z && v.w == v.w);
+                bad |= any_nan(v);
             }
         }
-        if (bad) {
-#pragma unroll 1
-            for (int e = 0; e < 64; ++e) {
-                const int64_t b = b0 + wn * 64 + 16 * (e >> 4) + l16, crq = rq0 + wm * 16 + (e >> 2 & 3) * 4 + lg;
-                if (b >= batch || crq >= n_rq) continue;
-                float *pe = part + ((int64_t)blockIdx.z * batch + b) * (n_rq * 4) + crq * 4 + (e & 3);
-                if (__builtin_isnan(*pe)) *pe = wgemm_plain_dot<WDT>(W, nblk, crq * 4 + (e & 3), blk_lo, blk_hi, x + b * ldx);
-            }
-        }
+        if (bad)
+            repair([&](int, int64_t b, int64_t crq, int) {
+                return part + ((int64_t)blockIdx.z * batch + b) * (n_rq * 4) + crq * 4;
+            });
         return;
     }
     // through LDS in TM / 64 passes of 64 weight rows, so that consecutive threads store consecutive outputs
     float *et = reinterpret_cast<float *>(smem);
-    for (int i = tid; i < TN; i += NT) et[i * kERow + 64] = xscale && b0 + i < batch ? xscale[b0 + i] : 1.0f;
 #pragma unroll
     for (int half = 0; half < TM / 64; ++half) {
         if (wm == half) {
+            bool bad = false;
+            auto at = [&](int t, int c) { return et + (wn * 64 + 16 * c + l16) * kERow + 16 * t + 4 * lg; };
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
                     float4 v;
                     v.x = acc[t][c][0]; v.y = acc[t][c][1]; v.z = acc[t][c][2]; v.w = acc[t][c][3];
-                    *reinterpret_cast<float4 *>(et + (wn * 64 + 16 * c + l16) * kERow + 16 * t + 4 * lg) = v;
+                    *reinterpret_cast<float4 *>(at(t, c)) = v;
+                    bad |= any_nan(v);
                 }
+            if (bad) repair([&](int t, int64_t, int64_t, int c) { return at(t, c); });
         }
         __syncthreads();
         const int64_t r0 = (rq0 + half * 16) * 4;
@@ -246,11 +271,7 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
                 const int64_t b = b0 + bl_, oo = r0 / 2 + o;
                 if (b >= batch || oo >= rows_out) continue;
                 const float *er = et + bl_ * kERow + (o >> 1) * 4 + (o & 1);
-                const float sc = et[bl_ * kERow + 64];
-                float g = er[0] * sc, u = er[2] * sc;
-                const int64_t row = r0 + (o >> 1) * 4 + (o & 1);
-                if (__builtin_isnan(g)) g = wgemm_plain_dot<WDT>(W, nblk, row, 0, nblk, x + b * ldx);
-                if (__builtin_isnan(u)) u = wgemm_plain_dot<WDT>(W, nblk, row + 2, 0, nblk, x + b * ldx);
+                const float g = er[0], u = er[2];
                 y[b * ldy + oo] = g / (1.0f + __expf(-g)) * u;
             }
         } else {
@@ -258,8 +279,7 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
                 const int bl_ = i >> 6, rr = i & 63;
                 const int64_t b = b0 + bl_, row = r0 + rr;
                 if (b >= batch || row >= rows_out) continue;
-                float v = et[bl_ * kERow + rr] * et[bl_ * kERow + 64];
-                if (__builtin_isnan(v)) v = wgemm_plain_dot<WDT>(W, nblk, row, 0, nblk, x + b * ldx);
+                float v = et[bl_ * kERow + rr];
                 if (bias) v += bias[row];
                 if constexpr (EPI == EPI_ACCUM) v += y[b * ldy + row];
                 y[b * ldy + row] = v;
