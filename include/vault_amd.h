@@ -144,8 +144,8 @@ int64_t vgx_qgemm_workspace_bytes(int64_t batch, int64_t rows, int64_t cols, int
  * epilogues, plus a caller workspace.  The activations (after the optional RMSNorm) enter as a bf16
  * hi + lo pair (2^-17 relative); weights, scales and the per-block fp32 accumulation are exact as in
  * the GEMV.  F32 weights run on fp32 MFMA (fp32 products and sums; no workspace); BF16 and F16 weights on
- * the 16-bit MFMA with the activations in pieces when a workspace of vgx_qgemm_workspace_bytes is given
- * (of any content; its tile counters stay untouched), else as F32.  No RMSNorm prologue for these three: norm_w must
+ * the 16-bit MFMA with the activations in exact pieces when a workspace of vgx_qgemm_workspace_bytes is given
+ * (of any content; its tile counters stay untouched) and the shape is not too small for it to pay, else as F32.  No RMSNorm prologue for these three: norm_w must
  * be NULL.  Replaces the chunk-prefill projections
  * (src/vault_v3_model.py:2051, 2095-2096 on [clen x d] blocks), batched decode projections, and the
  * segment scorer's fc1 over a chunk (:1224-1247). */

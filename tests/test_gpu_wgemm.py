@@ -17,11 +17,13 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dt", [codec.BF16, codec.F16])
 @pytest.mark.parametrize("rows,cols,batch,epi", [
     (13, 32, 8, "store"), (2, 64, 65, "swiglu"), (257, 96, 63, "accum"), (1030, 1536, 129, "store"),
-    (1536, 8960, 64, "accum"), (640, 2048, 1000, "swiglu"), (256, 256, 9, "edge"), (70, 512, 40, "strided")])
+    (1536, 8960, 64, "accum"), (640, 2048, 1000, "swiglu"), (256, 256, 9, "edge"), (70, 512, 40, "strided"),
+    (2100, 32, 2000, "store"), (2048, 32, 2048, "accum"), (1100, 256, 1030, "accum"), (2100, 480, 1030, "swiglu"),
+    (70, 544, 9, "edge"), (1024, 544, 1000, "store")])
 def test_wgemm_matches_oracle(dev, dt, rows, cols, batch, epi):
     """Tile edges (256 weight rows, 64 activation rows), one K block, K splits with a short last one, every
-    epilogue; "edge": weights and rows of extreme magnitudes (fp16 subnormals, rows of 1e-30 .. 1e30) and
-    non-finite activations; "strided": rows at an odd float offset and stride."""
+    epilogue, both sides of the line to the fp32 MFMA (few columns); "edge": weights and rows of extreme
+    magnitudes (fp16 subnormals, rows of 1e-30 .. 1e30) and non-finite activations; "strided": rows at an odd float offset and stride."""
     rng = np.random.default_rng(rows + cols + batch)
     mk = lambda seed: vlt3.quantize(dt, np.random.default_rng(seed).standard_normal((rows, cols)).astype(np.float32)
                                     * (1e-5 if epi == "edge" else 0.05))  # noqa: E731
@@ -84,10 +86,10 @@ def test_wgemm_leaves_the_tile_counters(dev, dt):
 
 
 @pytest.mark.parametrize("dt", [codec.BF16, codec.F16])
-@pytest.mark.parametrize("rows,cols,batch", [(70, 96, 9), (258, 1536, 70)])
+@pytest.mark.parametrize("rows,cols,batch", [(70, 96, 9), (258, 1536, 70), (33000, 480, 9)])
 @pytest.mark.parametrize("swiglu", [False, True])
 def test_wgemm_infinities(dev, dt, rows, cols, batch, swiglu):
-    """Infinite and NaN weights and activations (one K range and several): against activations of few bits, whose lower
+    """Infinite and NaN weights and activations (the fp32 MFMA, several K ranges, one): against activations of few bits, whose lower
     pieces are zero, against zeros, each other and ordinary elements.  An output is infinite or NaN where the float64
     product is, and within the usual bound elsewhere."""
     rng = np.random.default_rng(rows)

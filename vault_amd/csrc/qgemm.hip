@@ -662,9 +662,8 @@ __global__ __launch_bounds__(256, 3) void qgemm_tile_dma_kernel(const uint8_t *_
 }
 
 // ---------------------------------------------------------------------------------------------
-// F32 weights (the segment scorer's fc1, F32 model files), and BF16 / F16 weights of callers without a
-// workspace or past wgemm_tile_kernel's buffer ranges, for many activation
-// rows, 16-bit elements widened exactly to fp32 as they are fetched: fp32 MFMA
+// F32 weights (the segment scorer's fc1, F32 model files), and BF16 / F16 weights of few columns (wgemm_pays), of
+// callers without a workspace or past wgemm_tile_kernel's buffer ranges, for many activation rows, 16-bit elements widened exactly to fp32 as they are fetched: fp32 MFMA
 // (v_mfma_f32_16x16x4_f32), so products and sums stay fp32 as in the reference.  A workgroup of 4
 // waves owns 64 weight rows x 64 activation rows (each wave 32 x 32 as 2 x 2 tiles); per 32-wide
 // block of K the workgroup stages both 64 x 32 fp32 tiles in LDS (double-buffered, one barrier per
@@ -2428,6 +2427,18 @@ inline int64_t wgemm_bytes(int64_t batch, int64_t n_rq, int nblk) {
            part_bytes(wgemm_ksplit(n_rq, batch, nblk), batch, n_rq * 4);
 }
 
+// Whether wgemm_tile_kernel is ahead of f32gemm_tile_kernel for `tiles` 64 x 64 tiles of the latter.  Below 16 blocks
+// (no K splits) it waits out its pre-pass and one K range on few CUs, while the fp32 kernel is done after one round
+// of its tiles over the CUs.  Times fp32 | this, us, BF16 (F16): 64 columns 256 tiles 6.6 | 13, 512 tiles at 0.72
+// (0.66) of this, 1024 at 1.06 (0.97); 256 columns 256 tiles 13 | 17 (13 | 21), 512 at 1.05 (0.85), 1024 at 1.5
+// (1.26); 480 columns 1 to 256 tiles at 0.86-0.94 (0.64-0.71); 512 columns at 1.01-1.6 (0.85-1.24: behind with 129-256
+// tiles of whole batches, up to 640 columns); from 768 columns on 1.2 (1.07) at least.
+inline bool wgemm_pays(int dtype, int nblk, int64_t tiles, int64_t batch) {
+    const bool f16 = dtype == VGX_F16;
+    if (nblk < 16) return tiles > (nblk == 1 ? 1024 : nblk < 8 || f16 ? 512 : 256);
+    return !(f16 && nblk < 24 && batch > 64 && tiles > 128 && tiles <= 256);
+}
+
 template <int WDT>
 int wgemm_launch(const void *w_packed, int64_t rows, int64_t n_rq, int nblk, const float *x, int64_t ldx, int64_t batch,
                  const float *bias, float *y, int64_t ldy, int epilogue, void *workspace, hipStream_t st) {
@@ -2499,12 +2510,14 @@ int vgx_qgemm(int dtype, const void *w_packed, int64_t rows, int64_t cols, const
     const int64_t n_rq = rows4(rows_packed) / 4;
     if (dtype == VGX_F32 || dtype == VGX_BF16 || dtype == VGX_F16) {
         if (norm_w) return VGX_E_ARG;                 // plain weights: no fused RMSNorm on this path
-        // 16-bit weights on the 16-bit matrix cores when the caller brought the workspace and the operands
-        // fit the DMA's buffer ranges; without one (it is optional here) on the fp32 MFMA.  Gate/up | down
-        // of BF16 files at 8, 40, 333, 1024 rows: 107 -> 25, 108 -> 33, 243 -> 76, 591 -> 184 us | 472 ->
-        // 24, 474 -> 28, 462 -> 53, 467 -> 107 us: ahead at every batch size this entry takes
+        // 16-bit weights on the 16-bit matrix cores where that pays, the caller brought the workspace and the
+        // operands fit the DMA's buffer ranges; else (the workspace is optional here) on the fp32 MFMA.  Gate/up |
+        // down of BF16 files at 8, 40, 333, 1024 rows: 107 -> 25, 108 -> 33, 243 -> 76, 591 -> 184 us | 472 -> 24,
+        // 474 -> 28, 462 -> 53, 467 -> 107 us
+        const dim3 grid((unsigned)((n_rq + kFT / 4 - 1) / (kFT / 4)), (unsigned)((batch + kFT - 1) / kFT));
         const int64_t pbytes = kPlanes * split_plane_bytes(batch, cols);
-        if (dtype != VGX_F32 && workspace && (uintptr_t)workspace % 256 == 0 &&
+        if (dtype != VGX_F32 && wgemm_pays(dtype, nblk, (int64_t)grid.x * grid.y, batch) && workspace &&
+            (uintptr_t)workspace % 256 == 0 &&
             workspace_bytes >= wgemm_bytes(batch, n_rq, nblk) && n_rq * nblk * 256 < ((int64_t)1 << 31) &&
             pbytes < ((int64_t)1 << 31)) {
             if (dtype == VGX_BF16)
@@ -2514,7 +2527,6 @@ int vgx_qgemm(int dtype, const void *w_packed, int64_t rows, int64_t cols, const
                                          (hipStream_t)stream);
         }
         const void *wf = w_packed;
-        const dim3 grid((unsigned)((n_rq + kFT / 4 - 1) / (kFT / 4)), (unsigned)((batch + kFT - 1) / kFT));
         const bool vec = ((uintptr_t)x & 15) == 0 && ldx % 4 == 0;
         hipStream_t sf = (hipStream_t)stream;
 #define VGX_F32G(WDT, EPI, V) hipLaunchKernelGGL((f32gemm_tile_kernel<WDT, EPI, V>), grid, dim3(256), 0, sf, wf, n_rq, nblk, rows, x, ldx, batch, bias, y, ldy)
