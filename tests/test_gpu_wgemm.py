@@ -139,3 +139,37 @@ def test_wgemm_elements_keep_their_own_exponent(dev, dt, big):
     wf = codec.decode(dt, raw, rows, cols)
     y = ops.qlinear(ops.QWeight.from_blocks(dt, rows, cols, raw, dev), torch.from_numpy(x).to(dev)).cpu().numpy()
     assert np.all(np.abs(y - linalg.gemv(wf, x)) <= linalg.gemv_bound(wf, x, dt))
+
+
+@pytest.mark.parametrize("dt", [codec.BF16, codec.F16])
+@pytest.mark.parametrize("how", ["none", "short", "weights at 8 bytes"])
+@pytest.mark.parametrize("epi", [L.EPI_STORE, L.EPI_ACCUM, L.EPI_SWIGLU])
+def test_qgemm_16bit_weights_without_the_planes(dev, dt, how, epi):
+    """vgx_qgemm of 16-bit weights where the DMA tiles cannot run (no workspace, one without room for the partials, weights that are
+    not 16-byte aligned) runs on the fp32 MFMA: odd row counts, more rows and activations than a tile."""
+    lib, rng = L.load(), np.random.default_rng(4)
+    rows, cols, batch = (106 if epi == L.EPI_SWIGLU else 205), 1056, 70
+    mk = lambda: vlt3.quantize(dt, (rng.standard_normal((rows, cols)) * 0.05).astype(np.float32))  # noqa: E731
+    raws = [mk() for _ in range(2 if epi == L.EPI_SWIGLU else 1)]
+    w = ops.QWeight.gateup_from_blocks(dt, rows, cols, *raws, dev) if epi == L.EPI_SWIGLU else \
+        ops.QWeight.from_blocks(dt, rows, cols, raws[0], dev)
+    shift = torch.empty(w.packed.numel() + 8, dtype=torch.uint8, device=dev)
+    shift[8:] = w.packed
+    x, y0 = (rng.standard_normal((batch, n)).astype(np.float32) for n in (cols, rows))
+    xt, y = torch.from_numpy(x).to(dev), torch.from_numpy(y0).to(dev)
+    need = int(lib.vgx_qgemm_workspace_bytes(batch, rows, cols, epi))
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    size = {"none": 0, "short": 65536 + 3 * batch * cols * 2, "weights at 8 bytes": need}[how]
+    L.check(lib.vgx_qgemm(dt, shift.data_ptr() + 8 if size == need else w.packed.data_ptr(), rows, cols, xt.data_ptr(), cols,
+                          batch, None, 0.0, None, y.data_ptr(), rows, epi, ws.data_ptr() if size else None, size,
+                          torch.cuda.current_stream().cuda_stream), "vgx_qgemm")
+    assert int(ws.max()) == 0                                   # untouched
+    wf = [codec.decode(dt, r, rows, cols) for r in raws]
+    ref, bound = [linalg.gemv(f, x) for f in wf], [linalg.gemv_bound(f, x, dt) for f in wf]
+    if epi == L.EPI_SWIGLU:
+        out = linalg.swiglu(*ref)
+        tol = 1.1 * np.abs(ref[1]) * bound[0] + np.abs(ref[0]) * bound[1] + 1e-6 * np.abs(out) + 1e-30
+    else:
+        out = ref[0] + (y0 if epi == L.EPI_ACCUM else 0.0)
+        tol = bound[0] + np.abs(out) * 2e-7
+    assert np.all(np.abs(y.double().cpu().numpy() - out) <= tol)

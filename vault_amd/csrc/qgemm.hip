@@ -2511,13 +2511,13 @@ int vgx_qgemm(int dtype, const void *w_packed, int64_t rows, int64_t cols, const
     if (dtype == VGX_F32 || dtype == VGX_BF16 || dtype == VGX_F16) {
         if (norm_w) return VGX_E_ARG;                 // plain weights: no fused RMSNorm on this path
         // 16-bit weights on the 16-bit matrix cores where that pays, the caller brought the workspace and the
-        // operands fit the DMA's buffer ranges; else (the workspace is optional here) on the fp32 MFMA.  Gate/up |
+        // operands fit the DMA's buffer ranges and 16-byte pieces; else (the workspace is optional here) on the fp32 MFMA.  Gate/up |
         // down of BF16 files at 8, 40, 333, 1024 rows: 107 -> 25, 108 -> 33, 243 -> 76, 591 -> 184 us | 472 -> 24,
         // 474 -> 28, 462 -> 53, 467 -> 107 us
         const dim3 grid((unsigned)((n_rq + kFT / 4 - 1) / (kFT / 4)), (unsigned)((batch + kFT - 1) / kFT));
         const int64_t pbytes = kPlanes * split_plane_bytes(batch, cols);
         if (dtype != VGX_F32 && wgemm_pays(dtype, nblk, (int64_t)grid.x * grid.y, batch) && workspace &&
-            (uintptr_t)workspace % 256 == 0 &&
+            (uintptr_t)workspace % 256 == 0 && (uintptr_t)w_packed % 16 == 0 &&
             workspace_bytes >= wgemm_bytes(batch, n_rq, nblk) && n_rq * nblk * 256 < ((int64_t)1 << 31) &&
             pbytes < ((int64_t)1 << 31)) {
             if (dtype == VGX_BF16)
