@@ -272,9 +272,9 @@ int vgx_attn_prefill(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_bl
                      int64_t G, int64_t D, float scale, void *stream);
 
 /* vgx_attn_prefill with the planes of its fp32 K / V in a workspace (16-byte aligned, vgx_attn_prefill_planes_bytes of
- * the same blocks): each 64 keys of a kv group as fp16 hi + lo under a power of two, converted once per call instead
- * of by every workgroup that reads them (a smaller workspace, and calls that need 0 bytes, as bf16 K / V and few
- * keys, run as vgx_attn_prefill). */
+ * the same blocks): the three bf16 pieces, split once per call instead of by every workgroup that reads them, with the
+ * same results bit for bit (a smaller workspace, and calls that need 0 bytes, as bf16 K / V and few keys, run as
+ * vgx_attn_prefill). */
 int64_t vgx_attn_prefill_planes_bytes(int kv_dtype, const vgx_attn_block *blocks, int n_blocks, int64_t H, int64_t G);
 int vgx_attn_prefill_planes(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_block *blocks, int n_blocks,
                             int64_t H, int64_t G, int64_t D, float scale, void *workspace, int64_t workspace_bytes,

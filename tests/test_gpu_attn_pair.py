@@ -1,4 +1,4 @@
-"""GPU parity of the prefill attention over fp32 K / V held as scaled fp16 planes (vgx_attn_prefill_planes,
+"""GPU parity of the prefill attention over fp32 K / V held as bf16 planes (vgx_attn_prefill_planes,
 ops.attn_prefill without a Workspace) and of the bf16 tiles at one and two heads per group, against the
 float64 oracle.  Bars: those of test_gpu_attn_prefill.py (1e-5 fp32, 2e-3 bf16, values of order 1), times the
 magnitude of V where V is scaled."""
@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from oracle import attention as oatt
+from vault_amd import _lib as L
 from vault_amd import ops
 
 pytestmark = pytest.mark.gpu
@@ -41,7 +42,7 @@ def test_prefill_tiles_match_oracle(dev, H, G, T, lens, ws, kvdt):
 
 @pytest.mark.parametrize("ws", [False, True])
 def test_prefill_planes_scales(dev, ws):
-    """Powers of two per 64 keys: V of 2^-40 and zero in the first run (whose keys carry the weight of half of the
+    """Magnitudes far apart between key runs: V of 2^-40 and zero in the first run (whose keys carry the weight of half of the
     queries), 2^20 in the last; queries and keys of reciprocal magnitudes 2^+-30.  Bar: 1e-5 of the largest V that a
     query gives a weight of 2^-24 or more."""
     rng = np.random.default_rng(5)
@@ -78,3 +79,105 @@ def test_prefill_planes_share_runs(dev):
     got = go()
     assert not np.isfinite(got[460:, :4, 3]).any() and np.abs(got[:400] - ref[:400]).max() <= TOL32
     assert np.abs(got[400:, :, 4:] - ref[400:, :, 4:]).max() <= TOL32
+
+
+def _bits(q, runs, H, G, dev):
+    """vgx_attn_prefill itself: fp32 K / V split by every workgroup, no planes."""
+    out = torch.empty(q.shape, device=dev)
+    ra = (L.KVRun * 4)(*[L.KVRun(k.data_ptr(), v.data_ptr(), k.shape[1], k.stride(1), k.stride(0)) for k, v in runs])
+    arr = (L.AttnBlock * 1)(L.AttnBlock(q.data_ptr(), q.stride(0), q.stride(1), out.data_ptr(), out.stride(0),
+                                        out.stride(1), q.shape[0], 0, len(runs), ra))
+    L.check(L.load().vgx_attn_prefill(L.F32, L.BF16 if q.dtype == torch.bfloat16 else L.F32, L.F32, arr, 1, H, G, 128,
+                                      128 ** -0.5, torch.cuda.current_stream().cuda_stream), "vgx_attn_prefill")
+    return out
+
+
+@pytest.mark.parametrize("H,G", [(4, 4), (4, 2), (8, 2), (12, 2), (16, 2)])
+@pytest.mark.parametrize("qdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,lens", [(129, (64, 1, 128)), (2300, (65,)), (33, (500,)), (1, (200, 31, 95))])
+def test_prefill_planes_keep_the_bits(dev, H, G, qdt, T, lens):
+    """Planes or not, the same bits: K and V elements over twelve orders of magnitude, every launch shape."""
+    rng = np.random.default_rng(H + T)
+    runs = [tuple(_t(rng.standard_normal((G, n, 136)) * 10.0 ** rng.uniform(-6, 6, (G, n, 136)))[:, :, :128]
+                  for _ in range(2)) for n in lens + (T,)]
+    q, out = _t(rng.standard_normal((T, H, 128)), qdt), torch.empty(T, H, 128, device=dev)
+    ops.attn_prefill([{"q": q, "out": out, "runs": runs, "causal_base": 0}], H, G)
+    assert torch.equal(out, _bits(q, runs, H, G, dev))
+
+
+def test_prefill_planes_without_memory(dev, monkeypatch):
+    rng = np.random.default_rng(12)
+    q, k, v = (_t(rng.standard_normal(s)) for s in ((200, 8, 128), (2, 200, 128), (2, 200, 128)))
+    out, empty = torch.empty(200, 8, 128, device=dev), torch.empty
+
+    def full(*a, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError("no room")
+        return empty(*a, **kw)
+    monkeypatch.setattr(torch, "empty", full)
+    ops.attn_prefill([{"q": q, "out": out, "runs": [(k, v)], "causal_base": 0}], 8, 2)
+    monkeypatch.undo()
+    assert torch.equal(out, _bits(q, [(k, v)], 8, 2, dev))
+
+
+@pytest.mark.parametrize("x", [1e10, 1e30])
+@pytest.mark.parametrize("where", ["k", "v"])
+def test_prefill_future_keys_change_nothing(dev, x, where):
+    """A large element of a later key: queries before it keep their values (their bits, but for those whose wave of 16
+    queries reaches it, where the running max may move at another key)."""
+    rng = np.random.default_rng(8)
+    H, G, T, at = 8, 2, 300, 170
+    q, k, v = (_t(rng.standard_normal(s)) for s in ((T, H, 128), (G, T, 128), (G, T, 128)))
+
+    def go():
+        out = torch.empty(T, H, 128, device=dev)
+        ops.attn_prefill([{"q": q, "out": out, "runs": [(k, v)], "causal_base": 0}], H, G)
+        return out
+    before = go()
+    (k if where == "k" else v)[:, at, 5] = x
+    after = go()
+    assert torch.equal(before[:at // 16 * 16], after[:at // 16 * 16])
+    assert float((before - after)[:at].abs().max()) <= TOL32
+
+
+def test_prefill_unweighted_key_changes_nothing(dev):
+    """A key whose weight is zero, with V of 1e30 beside V of order 1 in the same 32 keys."""
+    rng = np.random.default_rng(9)
+    H, G, T = 12, 2, 200
+    q, k, v = (rng.standard_normal(s) for s in ((T, H, 128), (G, T, 128), (G, T, 128)))
+    q[:, :, 0], k[:, :, 0] = 20.0, 0.0
+    k[:, 3, 0], v[:, 3] = -1e4, 1e30
+    qt, kt, vt = _t(q), _t(k), _t(v)
+    out = torch.empty(T, H, 128, device=dev)
+    ops.attn_prefill([{"q": qt, "out": out, "runs": [(kt, vt)], "causal_base": 0}], H, G)
+    assert np.abs(out.double().cpu().numpy() - _ref(qt, [(kt, vt)]))[4:].max() <= TOL32
+
+
+def test_prefill_elements_keep_their_own_exponent(dev):
+    """Dims of a key, a value and a query of magnitudes far apart: V of 1e10 in one dim beside 1 in the others, and a
+    score made of one large query element on a small key element beside a large key element on none.  Bar: 1e-5 of
+    each dim's own magnitude."""
+    rng = np.random.default_rng(11)
+    H, G, T = 8, 2, 200
+    q, k, v = (rng.standard_normal(s) for s in ((T, H, 128), (G, T, 128), (G, T, 128)))
+    v[:, :, 7] *= 1e10
+    q[:, :, 3], k[:, :, 3] = q[:, :, 3] * 1e10, k[:, :, 3] * 1e-10
+    q[:, :, 4], k[:, :, 4] = 0.0, k[:, :, 4] * 1e10
+    qt, kt, vt = _t(q), _t(k), _t(v)
+    out = torch.empty(T, H, 128, device=dev)
+    ops.attn_prefill([{"q": qt, "out": out, "runs": [(kt, vt)], "causal_base": 0}], H, G)
+    err = np.abs(out.double().cpu().numpy() - _ref(qt, [(kt, vt)]))
+    assert err[:, :, 7].max() <= TOL32 * 1e10 and np.delete(err, 7, axis=2).max() <= TOL32
+
+
+@pytest.mark.parametrize("big", [2.0 ** 20, 2.0 ** 60, 2.0 ** 100])
+def test_prefill_zero_values_keep_their_weight(dev, big):
+    """Equal scores over 64 keys of zero V and keys of large V: the zeros hold their share of the softmax sum."""
+    rng = np.random.default_rng(10)
+    H, G, T = 4, 4, 150
+    q = torch.zeros(T, H, 128, device=dev)
+    runs = [(_t(rng.standard_normal((G, 64, 128))), torch.zeros(G, 64, 128, device=dev)),
+            (_t(rng.standard_normal((G, T, 128))), _t(rng.uniform(0.5, 1.0, (G, T, 128)) * big))]
+    out = torch.empty(T, H, 128, device=dev)
+    ops.attn_prefill([{"q": q, "out": out, "runs": runs, "causal_base": 0}], H, G)
+    assert np.abs(out.double().cpu().numpy() - _ref(q, runs)).max() <= TOL32 * big

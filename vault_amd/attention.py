@@ -6,7 +6,7 @@ src/vault_v3_model.py:812-863: q (B, H, L, D) post-RoPE, k / v (B, G, L, D) post
 i-1, causally to chunk i, and for i >= 2 to the first n_sink tokens re-rotated to the virtual
 positions (i-1)W - n_sink + j (clamped at 0; :805-809).  The attention runs in the MFMA prefill
 kernel (vgx_attn_prefill) in the dtype of k / v, as the reference's SDPA runs in its input dtype:
-bf16 K / V as they are, fp32 K / V as scaled fp16 hi + lo or three bf16 pieces (fp32-level results); other float
+bf16 K / V as they are, fp32 K / V as three bf16 pieces each (fp32-level results); other float
 dtypes take the fp32 path.  The sink keys are re-rotated on the GPU (vgx_rope_rotate) in fp32 with
 float32 angles, the reference's rope_cos_sin arithmetic (:777-782), and stored once in the K / V
 dtype (the reference rotates bf16 keys in bf16 arithmetic, :790-794, which rounds three times).
@@ -131,7 +131,7 @@ def block_sliding_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, w
             runs += [kb0 + o, vb0 + o, r1 - r0, ks[2], ks[1]]
             words += [qb0 + r0 * qs[2] * qe, qs[2], qs[1], ob0 + r0 * os_[2] * oe, os_[2], os_[1], r1 - r0, 0, nr]
             words += runs + none * (4 - nr) + none
-    ops.attn_prefill_words(words, kvdt, qq.dtype, out.dtype, H, G, D, D ** -0.5, q.device)
+    ops.attn_prefill_words(words, kvdt, qq.dtype, out.dtype, H, G, D, D ** -0.5, q.device, min(Lq, 2 * W) + S)
     return out if out.dtype == q.dtype else out.to(q.dtype)
 
 

@@ -1,5 +1,5 @@
-// Prefill attention on bf16 MFMA: blocks of queries over up to four key runs (sinks | segment
-// memory | previous chunk | current chunk), the last run causal.
+// Prefill attention on bf16 MFMA (fp32 operands in three bf16 pieces): blocks of queries over up to four
+// key runs (sinks | segment memory | previous chunk | current chunk), the last run causal.
 //
 // Reference semantics: block_sliding_attention (src/vault_v3_model.py:812-863, sinks re-rotated per
 // query chunk :805-809, 849-856) and the chunk-recurrent attention of _forward_chunk_recurrent
@@ -19,31 +19,28 @@
 //   O^T (dims x queries) += V^T P^T    A = V^T from LDS, B = P^T straight from the S^T accumulators
 //                                      as a bf16 hi + lo pair (two MFMAs): 8-bit probabilities alone
 //                                      exceed the bf16 attention bound when few keys carry the weight.
-// Staging.  K / V are copied into LDS by LDS DMA (buffer loads that
-// write LDS, no registers or VALU involved), double-buffered in 128-key tiles (fp32: 64-key tiles of the
-// fp16 planes below): the next tile's loads
-// leave right after the barrier that publishes the current one.  Both tiles keep the rows as they are
+// Staging.  K / V are copied into LDS by LDS DMA (buffer loads that write LDS, no registers or VALU involved),
+// double-buffered in 128-key tiles (fp32: 32-key tiles of the planes below): the next tile's loads leave right after
+// the barrier that publishes the current one.  Both tiles keep the rows as they are
 // in memory (256 bytes per key), each 16-byte piece p of row r stored at slot p ^ (r & 15), so the
 // 16-byte K reads of 16 rows and the transposed V reads stay free of bank conflicts; the V^T operand
 // comes from ds_read_b64_tr_b16, which hands lane i of a 16-lane group element i % 4 of the 8-byte
 // pieces that lanes i / 4 + 4 k address (k = 0..3): lane lq addresses key 4 lg + lq / 4, dims
 // 16 dt + 4 (lq % 4) .. + 3, and receives dim 16 dt + lq of keys 4 lg .. 4 lg + 3.
-// bf16 K and V stay bf16 end to end.  fp32 K and V with a workspace for planes: kv_pair_kernel writes them once per call as
-// fp16 hi + lo planes (22 bits or more) under a power of two per 64 keys and kv group; queries (a power of two
-// each) and probabilities are split the same way, and each product keeps hi x hi, hi x lo and lo x hi.  The K scale
-// multiplies the scores; the V scale enters the weights' exponent, so it is part of the running max, and is taken out
-// of the sum.  Three MFMAs per product and no conversions in the tile loop instead of six and the staging below:
-// two sequences of 2500 at 12 / 2 heads 348 -> 178 us, at 4 / 4 heads 885 -> 170 (the whole call);
-// relative error against 64 bits 4.4e-7 -> 3.5e-7.  At 3584 keys the kernel takes 76 us for 1024
-// queries (19.3 GFLOP, its MFMAs 23 us at peak): the chain scores -> softmax -> P V of three waves per SIMD and
-// 32 KB of LDS reads per wave and 32 keys bound it.
-// Without that workspace, for few keys, or with key ranges (vgx_attn_prefill_ws), each fp32 tile is loaded into registers during the previous tile's
-// math and stored into LDS as three bf16 planes (hi, mid, lo: 24 significant bits), K as is (padded rows), V
-// transposed; the fp32
-// queries and the probabilities are split the same way; each product keeps the six piece pairs of
-// order <= 2 (hi x hi, hi x mid, mid x hi, hi x lo, lo x hi, mid x mid) and drops those below 2^-24
-// of it, so scores and outputs carry fp32-level error (about 2^-22 relative) instead of the 2^-17 of
-// a hi + lo split.  In both products a lane of the 16 x 16 output owns
+// bf16 K and V stay bf16 end to end.  fp32 K and V enter as three bf16 planes (hi, mid, lo: 24 significant bits,
+// each element under its own exponent); the fp32 queries and the probabilities are split the same way; each
+// product keeps the six piece pairs of order <= 2 (hi x hi, hi x mid, mid x hi, hi x lo, lo x hi, mid x mid) and
+// drops those below 2^-24 of it, so scores and outputs carry fp32-level error (about 2^-22 relative) instead of
+// the 2^-17 of a hi + lo split.  With a workspace for them the planes are written once per call (kv_planes_kernel) and
+// staged by LDS DMA; without it, for few keys, or with key ranges (vgx_attn_prefill_ws) every workgroup loads
+// its fp32 tiles into registers during the previous tile's math, splits them and stores the planes into LDS, K as
+// is (padded rows), V transposed: the same pieces in the same order, so the same bits: two sequences
+// of 2500 at 12 / 2 heads 349 -> 255 us for the whole call, 1024 queries over 3584 keys at 4 / 4 heads 597 -> 196.  Six
+// products of 64.6 million pairs x 128 dims x 2 are 198 GFLOP there, 165 us at the 1.2 PFLOP/s of a large bf16
+// product on this card; 25 us are the planes and the sinks.  What it took beside the DMA: each wave's loads of a
+// tile a fixed set of a few instructions (272 -> 255 us; at four waves a workgroup 255 -> 196), the operands of the next
+// 32 dims read while this one's are multiplied (266 -> 255, 229 -> 196).
+// In both products a lane of the 16 x 16 output owns
 // one query column, so the online-softmax state (running max, rescale of O) is lane-local; the max
 // over a query's keys needs two cross-lane steps.  The K-dimension slots of A and B are assigned the
 // same way in each product (lane group lg holds slots 8 lg .. 8 lg + 7 of both operands), which is
@@ -59,7 +56,6 @@ using namespace vgx;
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kD = 128;             // head dim (the kernel is specialised for 128)
@@ -84,18 +80,11 @@ __device__ __forceinline__ T sel4(int i, T a0, T a1, T a2, T a3) {
 }
 
 struct RunArgs {
-    const void *k;     // bf16 or fp32 rows; fp16 pair planes: the run's first plane
-    const void *v;     // fp16 pair planes: the run's PairScale entries
+    const void *k;     // bf16 or fp32 rows; planes: the run's first plane
+    const void *v;
     int64_t len;
-    int64_t rstride;   // elements between consecutive keys; fp16 pair planes: rows per kv group
+    int64_t rstride;   // elements between consecutive keys; planes: rows per kv group
     int64_t gstride;   // elements between kv groups
-};
-
-// Power-of-two scales of kPairKeys keys of one kv group: the plane holds 2^-log2 x the value.
-constexpr int kPairKeys = 64;
-struct PairScale {
-    float k;           // 2^log2 of the K rows
-    float v_log2;      // log2 of the V rows' scale
 };
 
 struct BlockArgs {
@@ -136,111 +125,72 @@ struct PrefillArgs {
 // the running max and sum.
 __host__ __device__ constexpr int prefill_slot_floats(int waves, int nqt) { return waves * nqt * (8 * 256 + 32); }
 
-constexpr float kPairBoost = 6.0f;  // log2 of the weights' scale: at most 2^(kLazyMax + 6) < 65504 in fp16
-
-template <bool F16>
 __device__ __forceinline__ f32x4_t mfma16(bf16x8_t x, bf16x8_t y, f32x4_t c) {
-    if constexpr (F16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, x), __builtin_bit_cast(f16x8_t, y), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ float exp2i(int k) { return __uint_as_float((uint32_t)(k + 127) << 23); }   // |k| <= 126
-__device__ __forceinline__ float finite_abs(float x) { return __builtin_isfinite(x) ? fabsf(x) : 0.0f; }
-// k with 2^k mx in [2^14, 2^15), at most 100 (also for mx = 0: zero V rows then weigh nothing against the others in
-// the running max), so that sums of 2^k x probabilities stay in the fp32 range
-__device__ __forceinline__ int pair_exponent(float mx) { return min(100, 14 + 127 - (int)(__float_as_uint(mx) >> 23)); }
-// hi = fp16(a, b), lo = fp16(a - hi_a, b - hi_b) (0 where a, b is not finite)
-__device__ __forceinline__ void split_f16x2(float a, float b, uint32_t &hi, uint32_t &lo) {
-    hi = pack_f16x2(a, b);
-    const auto h = __builtin_bit_cast(vgx_f16x2_t, hi);
-    lo = pack_f16x2(a - (float)h[0], b - (float)h[1]);
-}
-
-// fp32 K / V runs as fp16 hi + lo planes, so that the attention kernel stages them by LDS DMA and needs three
-// MFMAs per product instead of the six of three bf16 planes.  Each kPairKeys keys of a kv group share a power
-// of two per operand (largest |element| in [2^14, 2^15)), so both pieces are normal fp16 numbers for every
-// element above 2^-28 of it, and the pair holds 22 bits or more.  A non-finite element is left
-// out of the scale and keeps its value in hi with a zero lo.
-struct PairRun {
+// fp32 K / V runs as three bf16 planes each, so that the attention kernel stages them by LDS DMA instead of
+// converting every tile in every workgroup that reads it.
+struct PlaneRun {
     const float *k, *v;
     int64_t len, rstride, gstride;
-    int64_t rows;              // len rounded up to kPairKeys
-    uint16_t *planes;          // K hi, K lo, V hi, V lo: [G][rows][kD] each
-    PairScale *scale;          // [G][rows / kPairKeys]
+    uint16_t *planes;          // K hi, K mid, K lo, V hi, V mid, V lo: [G][len][kD] each
     int wg0;                   // first workgroup of this run
 };
-constexpr int kMaxPairRuns = 4 * kMaxBlocks;
-struct PairArgs {
-    PairRun run[kMaxPairRuns];
+constexpr int kMaxPlaneRuns = 4 * kMaxBlocks;
+constexpr int kPlaneRows = 64;          // rows per workgroup of the conversion
+struct PlaneArgs {
+    PlaneRun run[kMaxPlaneRuns];
     int n_runs, G;
 };
 
-// One workgroup per (kPairKeys keys, kv group, K or V).
-__global__ __launch_bounds__(256) void kv_pair_kernel(PairArgs a) {
+// One workgroup per (kPlaneRows keys, kv group, K or V): a float4 per lane and row, 32 lanes a row.  Bound by its
+// reads and writes (4 + 6 bytes per element).
+__global__ __launch_bounds__(256) void kv_planes_kernel(PlaneArgs a) {
     int ri = 0;
     for (int i = 1; i < a.n_runs; ++i)
         if (a.run[i].wg0 <= (int)blockIdx.x) ri = i;
-    const PairRun &R = a.run[ri];
+    const PlaneRun &R = a.run[ri];
     const int local = blockIdx.x - R.wg0, isv = local & 1, g = (local >> 1) % a.G, grp = (local >> 1) / a.G;
-    const int64_t j0 = (int64_t)grp * kPairKeys;
+    const int64_t j0 = (int64_t)grp * kPlaneRows;
     const float *src = (isv ? R.v : R.k) + (int64_t)g * R.gstride;
-    constexpr int IT = kPairKeys * kD / 4 / 256;
+    constexpr int IT = kPlaneRows * kD / 4 / 256;
     const int col = threadIdx.x & 31, row0 = threadIdx.x >> 5;
     float4 x[IT];
-    float mx = 0.0f;
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
         const int64_t j = j0 + row0 + 8 * i;
-        x[i] = j < R.len ? *reinterpret_cast<const float4 *>(src + j * R.rstride + 4 * col) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (j < R.len) x[i] = *reinterpret_cast<const float4 *>(src + j * R.rstride + 4 * col);
     }
-#pragma unroll
-    for (int i = 0; i < IT; ++i)
-        mx = fmaxf(fmaxf(fmaxf(mx, finite_abs(x[i].x)), finite_abs(x[i].y)), fmaxf(finite_abs(x[i].z), finite_abs(x[i].w)));
-    for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
-    __shared__ float wm[4];
-    if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    const int k = pair_exponent(fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3])));
-    const float sc = exp2i(k);
-    if (threadIdx.x == 0) {
-        PairScale *e = R.scale + (int64_t)g * (R.rows / kPairKeys) + grp;
-        if (isv) e->v_log2 = (float)-k;
-        else e->k = exp2i(-k);
-    }
-    const int64_t ps = (int64_t)a.G * R.rows * kD;
-    uint16_t *hp = R.planes + (isv ? 2 * ps : 0) + ((int64_t)g * R.rows + j0) * kD;
+    const int64_t ps = (int64_t)a.G * R.len * kD;
+    uint16_t *hp = R.planes + (isv ? 3 * ps : 0) + (int64_t)g * R.len * kD;
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-        const int row = row0 + 8 * i;
-        uint2 hi, lo;
-        const float e[4] = {x[i].x * sc, x[i].y * sc, x[i].z * sc, x[i].w * sc};
-        split_f16x2(e[0], e[1], hi.x, lo.x);
-        split_f16x2(e[2], e[3], hi.y, lo.y);
-        if (!__builtin_isfinite(e[0])) lo.x &= 0xFFFF0000u;
-        if (!__builtin_isfinite(e[1])) lo.x &= 0xFFFFu;
-        if (!__builtin_isfinite(e[2])) lo.y &= 0xFFFF0000u;
-        if (!__builtin_isfinite(e[3])) lo.y &= 0xFFFFu;
-        *reinterpret_cast<uint2 *>(hp + row * kD + 4 * col) = hi;
-        *reinterpret_cast<uint2 *>(hp + ps + row * kD + 4 * col) = lo;
+        const int64_t j = j0 + row0 + 8 * i;
+        if (j >= R.len) continue;
+        uint2 hw, mw, lw;
+        split3_bf16x2(x[i].x, x[i].y, hw.x, mw.x, lw.x);
+        split3_bf16x2(x[i].z, x[i].w, hw.y, mw.y, lw.y);
+        uint16_t *p = hp + j * kD + 4 * col;
+        *reinterpret_cast<uint2 *>(p) = hw;
+        *reinterpret_cast<uint2 *>(p + ps) = mw;
+        *reinterpret_cast<uint2 *>(p + 2 * ps) = lw;
     }
 }
 
 template <int GRP, bool QSPLIT, int NQT, bool KF, int QW, bool DMA, int KT>
 __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs a) {
     constexpr int kQTile = 16 * NQT * QW;
-    constexpr bool PAIR = KF && DMA;                // fp32 K / V as the fp16 hi + lo planes of kv_pair_kernel
+    constexpr bool PLANES = KF && DMA;              // fp32 K / V as the bf16 planes of kv_planes_kernel
     constexpr int VROW = KT + 8;                    // LDS row of V^T, bf16 (16 bytes of padding)
-    constexpr int NP = PAIR ? 2 : KF ? 3 : 1;       // 16-bit planes per K / V operand
-    constexpr int NQP = QSPLIT ? (KF && !PAIR ? 3 : 2) : 1;  // 16-bit pieces per query
-    constexpr int NPP = KF && !PAIR ? 3 : 2;        // 16-bit pieces per probability
-    constexpr int ORD = KF && !PAIR ? 2 : 1;        // products of pieces i x j kept when i + j <= ORD
-    constexpr int ESZ = KF && !PAIR ? 4 : 2;        // bytes per staged K / V element in memory
+    constexpr int NP = KF ? 3 : 1;       // 16-bit planes per K / V operand
+    constexpr int NQP = QSPLIT ? (KF ? 3 : 2) : 1;  // 16-bit pieces per query
+    constexpr int NPP = KF ? 3 : 2;        // 16-bit pieces per probability
+    constexpr int ORD = KF ? 2 : 1;        // products of pieces i x j kept when i + j <= ORD
+    constexpr int ESZ = KF && !DMA ? 4 : 2;        // bytes per staged K / V element in memory
     constexpr int STAGE_E = 2 * NP * KT * kD;       // DMA: elements per stage
     constexpr int CH = 32;                          // keys per softmax step
     static_assert(KF || DMA, "bf16 K / V are staged by LDS DMA");
-    static_assert(!PAIR || KT == kPairKeys, "one scale per tile");
     __shared__ __align__(16) uint16_t ks[DMA ? 2 * STAGE_E : NP * KT * kKRow];   // DMA: [stage][K planes, V planes][key][dim]
     __shared__ __align__(16) uint16_t vt[DMA ? 8 : NP * kD * VROW];
 
@@ -267,77 +217,36 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
     // Q^T fragments (bf16): query t0 + 16 qt + lq, dims 32 kc + 8 lg .. + 7; fp32 queries as NQP
     // pieces: hi = bf16(q), then bf16 of what is left (lo, or mid and lo).
     bf16x8_t qf[NQP][NQT][4];
-    float qinv[NQT];                                // PAIR: 2^-k of the query's scale
-    if constexpr (PAIR) {
-        // fp16 pieces of the query scaled by a power of two (largest element in [2^14, 2^15))
 #pragma unroll
-        for (int qt = 0; qt < NQT; ++qt) {
-            const int64_t t = tw + qt * 16 + lq;
-            float e[4][8], mx = 0.0f;
+    for (int qt = 0; qt < NQT; ++qt) {
+        const int64_t t = tw + qt * 16 + lq;
 #pragma unroll
-            for (int kc = 0; kc < 4; ++kc) {
-                const int64_t at = t * B.ldq + h * B.q_hstride + kc * 32 + lg * 8;
-                if (t >= B.n_q) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) e[kc][i] = 0.0f;
-                } else if constexpr (QSPLIT) {
-                    const float *qp = static_cast<const float *>(B.q) + at;
+        for (int kc = 0; kc < 4; ++kc) {
+            const int d0 = kc * 32 + lg * 8;
+            uint32_t pw[NQP][4];
+            if (t < B.n_q) {
+                if constexpr (!QSPLIT) {
+                    const uint4 w = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(B.q) + t * B.ldq + h * B.q_hstride + d0);
+                    pw[0][0] = w.x; pw[0][1] = w.y; pw[0][2] = w.z; pw[0][3] = w.w;
+                } else {
+                    const float *qp = static_cast<const float *>(B.q) + t * B.ldq + h * B.q_hstride + d0;
                     const float4 x0 = reinterpret_cast<const float4 *>(qp)[0], x1 = reinterpret_cast<const float4 *>(qp)[1];
-                    e[kc][0] = x0.x; e[kc][1] = x0.y; e[kc][2] = x0.z; e[kc][3] = x0.w;
-                    e[kc][4] = x1.x; e[kc][5] = x1.y; e[kc][6] = x1.z; e[kc][7] = x1.w;
-                } else {
-                    const uint4 w = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(B.q) + at);
-                    const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+                    const float e[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) e[kc][i] = bf16_bits_to_float(ww[i / 2] >> (i & 1) * 16);
-                }
-#pragma unroll
-                for (int i = 0; i < 8; ++i) mx = fmaxf(mx, finite_abs(e[kc][i]));
-            }
-            const int k = pair_exponent(xor32_max(xor16_max(mx)));
-            qinv[qt] = exp2i(-k);
-            const float sc = exp2i(k);
-#pragma unroll
-            for (int kc = 0; kc < 4; ++kc) {
-                uint32_t hi[4], lo[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) split_f16x2(e[kc][2 * i] * sc, e[kc][2 * i + 1] * sc, hi[i], lo[i]);
-                qf[0][qt][kc] = __builtin_bit_cast(bf16x8_t, make_uint4(hi[0], hi[1], hi[2], hi[3]));
-                if constexpr (NQP == 2) qf[NQP - 1][qt][kc] = __builtin_bit_cast(bf16x8_t, make_uint4(lo[0], lo[1], lo[2], lo[3]));
-            }
-        }
-    } else {
-#pragma unroll
-        for (int qt = 0; qt < NQT; ++qt) {
-            const int64_t t = tw + qt * 16 + lq;
-#pragma unroll
-            for (int kc = 0; kc < 4; ++kc) {
-                const int d0 = kc * 32 + lg * 8;
-                uint32_t pw[NQP][4];
-                if (t < B.n_q) {
-                    if constexpr (!QSPLIT) {
-                        const uint4 w = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(B.q) + t * B.ldq + h * B.q_hstride + d0);
-                        pw[0][0] = w.x; pw[0][1] = w.y; pw[0][2] = w.z; pw[0][3] = w.w;
-                    } else {
-                        const float *qp = static_cast<const float *>(B.q) + t * B.ldq + h * B.q_hstride + d0;
-                        const float4 x0 = reinterpret_cast<const float4 *>(qp)[0], x1 = reinterpret_cast<const float4 *>(qp)[1];
-                        const float e[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            if constexpr (NQP == 3) split3_bf16x2(e[2 * i], e[2 * i + 1], pw[0][i], pw[1][i], pw[2][i]);
-                            else split_bf16x2(e[2 * i], e[2 * i + 1], pw[0][i], pw[NQP - 1][i]);
-                        }
+                    for (int i = 0; i < 4; ++i) {
+                        if constexpr (NQP == 3) split3_bf16x2(e[2 * i], e[2 * i + 1], pw[0][i], pw[1][i], pw[2][i]);
+                        else split_bf16x2(e[2 * i], e[2 * i + 1], pw[0][i], pw[NQP - 1][i]);
                     }
-                } else {
-#pragma unroll
-                    for (int pp = 0; pp < NQP; ++pp)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) pw[pp][i] = 0;
                 }
+            } else {
 #pragma unroll
                 for (int pp = 0; pp < NQP; ++pp)
-                    qf[pp][qt][kc] = __builtin_bit_cast(bf16x8_t, make_uint4(pw[pp][0], pw[pp][1], pw[pp][2], pw[pp][3]));
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) pw[pp][i] = 0;
             }
+#pragma unroll
+            for (int pp = 0; pp < NQP; ++pp)
+                qf[pp][qt][kc] = __builtin_bit_cast(bf16x8_t, make_uint4(pw[pp][0], pw[pp][1], pw[pp][2], pw[pp][3]));
         }
     }
 
@@ -357,16 +266,16 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
     const int64_t cbase = B.causal_base;
     int64_t rlen[4];
     const char *rkp[4], *rvp[4];
-    int rrs[4];                                    // PAIR: bytes between planes / 256
+    int rrs[4];                                    // bytes between keys; planes: between planes, in rows
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const RunArgs &R = B.run[i];
         int64_t n = i < n_runs ? R.len : 0;
         if (i == n_runs - 1 && cbase >= 0) n = min(n, cbase + t0 + kQTile);   // the rest is in every query's future
         rlen[i] = n;
-        if constexpr (PAIR) {
+        if constexpr (PLANES) {
             rkp[i] = static_cast<const char *>(R.k) + (int64_t)g * R.rstride * (kD * 2);
-            rvp[i] = static_cast<const char *>(R.v) + (int64_t)g * (R.rstride / kPairKeys) * sizeof(PairScale);
+            rvp[i] = nullptr;
             rrs[i] = (int)R.rstride * a.G;
             continue;
         }
@@ -409,27 +318,7 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
             }
         }
     };
-    PairScale tsc{1.0f, 0.0f};                     // PAIR: the scales of the tile in flight
     auto issue = [&](int r, int64_t j0, int buf) {
-        if constexpr (PAIR) {
-            constexpr int RB = kD * 2;
-            const char *p0 = sel4(r, rkp[0], rkp[1], rkp[2], rkp[3]) + j0 * RB;
-            const int64_t ps = (int64_t)sel4(r, rrs[0], rrs[1], rrs[2], rrs[3]) * RB;
-            const int lim = (int)min<int64_t>(run_len(r) - j0, KT);
-            tsc = reinterpret_cast<const PairScale *>(sel4(r, rvp[0], rvp[1], rvp[2], rvp[3]))[j0 / kPairKeys];
-            dma_rsrc_t rs[4];                       // K hi, K lo, V hi, V lo
-#pragma unroll
-            for (int p = 0; p < 4; ++p) rs[p] = dma_rsrc(p0 + p * ps, (uint32_t)(lim * RB));
-            uint8_t *base = reinterpret_cast<uint8_t *>(ks) + buf * (STAGE_E * 2);
-            const int sub = lane >> 4, slot = lane & 15;
-            for (int i = wave; i < KT / 4; i += NT / 64) {      // 4 rows of each plane
-                const int row = 4 * i + sub;
-                const uint32_t off = (uint32_t)(row * RB + ((slot ^ (row & 15)) << 4));
-#pragma unroll
-                for (int p = 0; p < 4; ++p) dma16(rs[p], off, base + (p * KT + 4 * i) * RB);
-            }
-            return;
-        }
         const int64_t n = run_len(r);
         const int rs = sel4(r, rrs[0], rrs[1], rrs[2], rrs[3]);
         const char *kb = sel4(r, rkp[0], rkp[1], rkp[2], rkp[3]) + j0 * rs;
@@ -444,6 +333,42 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
             dma16(isv ? vrs : krs, (uint32_t)(row * rs + ((slot ^ (row & 15)) << 4)),
                   base + (isv ? KT * kD * 2 : 0) + rb * kD * 2);
         }
+    };
+    // Planes: the tile in flight as 6 planes x 8 loads of 4 rows, split over the waves so that what changes between the
+    // loads of a wave is a constant: two waves a plane (12), one (6), or every plane by every wave (8 and 4).
+    // Its run's addresses are kept between tiles.
+    constexpr int RB = kD * 2, NWV = NT / 64, NLD = 2 * NP * KT / 4 / NWV;
+    static_assert(!PLANES || (2 * NP == 6 && KT == 32 && (NWV == 4 || NWV == 6 || NWV == 8 || NWV == 12)), "loads per wave");
+    const char *pl_at = nullptr;
+    int64_t pl_stride = 0;
+    int pl_left = 0;
+    const int pl_sub = NWV == 12 ? wave >> 1 : NWV == 6 ? wave : 0;             // first plane of the wave
+    const int pl_row = NWV == 12 ? 16 * (wave & 1) : NWV == 6 ? 0 : 4 * wave;   // its first row
+    // this lane's byte in the wave's first rows; rows 4 i further on, the piece's slot changes by an XOR with 4 i
+    const int pl_off = (pl_row + (lane >> 4)) * RB + (((lane & 15) ^ ((pl_row + (lane >> 4)) & 15)) << 4);
+    auto plane_run = [&](int r, int64_t j0) {
+        pl_at = sel4(r, rkp[0], rkp[1], rkp[2], rkp[3]) + j0 * RB;
+        pl_stride = (int64_t)sel4(r, rrs[0], rrs[1], rrs[2], rrs[3]) * RB;
+        pl_left = (int)(run_len(r) - j0);
+    };
+    auto issue_planes = [&](int buf) {
+        const uint32_t bytes = (uint32_t)min(pl_left, KT) * RB;
+        uint8_t *base = reinterpret_cast<uint8_t *>(ks) + buf * (STAGE_E * 2) + (pl_sub * KT + pl_row) * RB;
+        const char *at = pl_at + pl_sub * pl_stride;
+        dma_rsrc_t rs = dma_rsrc(at, bytes);
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+            // rows 4 i on (12 and 6 waves), plane i on (8), 16 rows and then the plane on (4)
+            if (NWV == 12 || NWV == 6) {
+                dma16(rs, (pl_off ^ (i & 3) << 6) + 4 * i * RB, base + 4 * i * RB);
+            } else {
+                const int p = NWV == 8 ? i : i >> 1, half = NWV == 8 ? 0 : i & 1;
+                if (p > 0 && !half) rs = dma_rsrc(at += pl_stride, bytes);
+                dma16(rs, pl_off + half * 16 * RB, base + (p * KT + half * 16) * RB);
+            }
+        }
+        pl_at += KT * RB;
+        pl_left -= KT;
     };
     auto stage = [&]() {
 #pragma unroll
@@ -507,8 +432,12 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
     }
     if (todo == 0) r = n_runs;
     int buf = 0;
-    float kscale = 1.0f, vlog = 0.0f, vinv = 1.0f;  // PAIR: 2^log2 of the tile's K, log2 and 2^-log2 of its V
-    if constexpr (DMA) {
+    if constexpr (PLANES) {
+        if (r < n_runs) {
+            plane_run(r, j0);
+            issue_planes(0);
+        }
+    } else if constexpr (DMA) {
         if (r < n_runs) issue(r, j0, 0);
     } else {
         if (r < n_runs) fetch(r, j0);
@@ -527,12 +456,14 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
             // this tile's loads landed (each wave waits for its own, the barrier for every wave's), and
             // every wave is done with the other stage: the next tile's loads go there
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if constexpr (PAIR) {
-                kscale = tsc.k * sl2;
-                vlog = tsc.v_log2;
-                vinv = __builtin_amdgcn_exp2f(-vlog);
+            if constexpr (PLANES) {
+                if (rn < n_runs) {
+                    if (rn != r) plane_run(rn, jn);
+                    issue_planes(buf ^ 1);
+                }
+            } else {
+                if (rn < n_runs) issue(rn, jn, buf ^ 1);
             }
-            if (rn < n_runs) issue(rn, jn, buf ^ 1);
         } else {
             __syncthreads();
             stage();
@@ -547,6 +478,46 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
             for (int qt = 0; qt < NQT; ++qt)
 #pragma unroll
                 for (int s = 0; s < NS; ++s) sc[qt][s] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (PLANES) {
+                // the operands of the next 32 dims are read while this one's are multiplied (the order that the
+                // scheduling groups below ask for; left to itself the compiler waits for each read)
+                bf16x8_t kf[2][NP][NS];
+                auto load = [&](int kc, bf16x8_t (&f)[NP][NS]) {
+#pragma unroll
+                    for (int pk = 0; pk < NP; ++pk)
+#pragma unroll
+                        for (int s = 0; s < NS; ++s)
+                            f[pk][s] = *reinterpret_cast<const bf16x8_t *>(kst + (pk * KT + c + 16 * s + lq) * (kD * 2) +
+                                                                           (((kc * 4 + lg) ^ lq) << 4));
+                };
+                load(0, kf[0]);
+#pragma unroll
+                for (int kc = 0; kc < 4; ++kc) {
+                    if (kc < 3) load(kc + 1, kf[(kc + 1) & 1]);
+#pragma unroll
+                    for (int pk = 0; pk < NP; ++pk)
+#pragma unroll
+                        for (int qp = 0; qp < NQP; ++qp) {
+                            if (pk + qp > ORD) continue;
+#pragma unroll
+                            for (int s = 0; s < NS; ++s)
+#pragma unroll
+                                for (int qt = 0; qt < NQT; ++qt)
+                                    sc[qt][s] = mfma16(kf[kc & 1][pk][s], qf[qp][qt][kc], sc[qt][s]);
+                        }
+                }
+                __builtin_amdgcn_sched_group_barrier(0x100, NP * NS, 0);
+#pragma unroll
+                for (int kc = 0; kc < 3; ++kc) {
+#pragma unroll
+                    for (int i = 0; i < NP * NS; ++i) {
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x008, NQP == 1 ? 1 : 2, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_group_barrier(0x008, 12, 0);
+                return;
+            }
 #pragma unroll
             for (int kc = 0; kc < 4; ++kc) {
 #pragma unroll
@@ -563,18 +534,17 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
                     }
 #pragma unroll
                     for (int qp = 0; qp < NQP; ++qp) {
-                        if (pk + qp > ORD) continue;      // below 2^-(8 (ORD + 1)) of the product (PAIR: 2^-24)
+                        if (pk + qp > ORD) continue;      // below 2^-(8 (ORD + 1)) of the product
 #pragma unroll
                         for (int s = 0; s < NS; ++s)
 #pragma unroll
                             for (int qt = 0; qt < NQT; ++qt)
-                                sc[qt][s] = mfma16<PAIR>(af[s], qf[qp][qt][kc], sc[qt][s]);
+                                sc[qt][s] = mfma16(af[s], qf[qp][qt][kc], sc[qt][s]);
                     }
                 }
             }
         };
-        auto finish = [&](int c, f32x4_t (&sc)[NQT][NS]) {
-            bf16x8_t pf[NPP][NQT][NS / 2];
+        auto softmax = [&](int c, f32x4_t (&sc)[NQT][NS], bf16x8_t (&pf)[NPP][NQT][NS / 2]) {
             // step fully visible to all of the wave's queries: no per-score mask
             const bool full = j0 + c + CH <= n && (!causal || j0 + c + CH - 1 <= cbase + tw);
             // the biased run of a biased head: its bias (log2 units) is added to the chunk's scores
@@ -585,17 +555,15 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
 #pragma unroll
             for (int qt = 0; qt < NQT; ++qt) {
                 float v[4 * NS];
-                float ssc = sl2;
-                if constexpr (PAIR) ssc = kscale * qinv[qt];
                 if (full) {
 #pragma unroll
-                    for (int i = 0; i < 4 * NS; ++i) v[i] = sc[qt][i / 4][i % 4] * ssc;
+                    for (int i = 0; i < 4 * NS; ++i) v[i] = sc[qt][i / 4][i % 4] * sl2;
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4 * NS; ++i) {
                         const int kk = i / 4 * 16 + lg * 4 + i % 4;        // key within the step
                         const bool vis = kk < klim && (!causal || kbase + kk <= qt * 16 + lq);
-                        v[i] = vis ? sc[qt][i / 4][i % 4] * ssc : -INFINITY;
+                        v[i] = vis ? sc[qt][i / 4][i % 4] * sl2 : -INFINITY;
                     }
                 }
                 if (biased) {
@@ -610,10 +578,9 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
 #pragma unroll
                 for (int i = 1; i < 4 * NS; ++i) mt = fmaxf(mt, v[i]);
                 mt = xor32_max(xor16_max(mt));
-                if constexpr (PAIR) mt += vlog;
-                // The reference max m (log2 units; PAIR: of score + log2 of the V scale) moves only when a
-                // score exceeds it by more than kLazyMax: probabilities then stay below 2^kLazyMax, and O
-                // and the sum are rescaled far less often than the running max changes.
+                // The reference max m moves only when a score exceeds it by more than kLazyMax
+                // (log2 units): probabilities then stay below 2^kLazyMax, and O and the sum are
+                // rescaled far less often than the running max changes.
                 if (__ballot(mt > m[qt] + kLazyMax)) {
                     const float mn = fmaxf(m[qt], mt);
                     const float corr = __builtin_amdgcn_exp2f(m[qt] - mn);
@@ -622,12 +589,10 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
 #pragma unroll
                     for (int dt = 0; dt < 8; ++dt) o[qt][dt] *= corr;
                 }
-                // PAIR: the weights carry the V scale and 2^kPairBoost, so that the lo pieces stay normal
-                const float mn = PAIR ? m[qt] - (vlog + kPairBoost) : m[qt];
                 float ps = 0.0f, pv[4 * NS];
 #pragma unroll
                 for (int i = 0; i < 4 * NS; ++i) {
-                    pv[i] = __builtin_amdgcn_exp2f(v[i] - mn);
+                    pv[i] = __builtin_amdgcn_exp2f(v[i] - m[qt]);
                     ps += pv[i];
                 }
 #pragma unroll
@@ -636,8 +601,7 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const float x = pv[8 * s2 + 2 * i], y = pv[8 * s2 + 2 * i + 1];
-                        if constexpr (PAIR) split_f16x2(x, y, pw[0][i], pw[1][i]);
-                        else if constexpr (NPP == 3) split3_bf16x2(x, y, pw[0][i], pw[1][i], pw[2][i]);
+                        if constexpr (NPP == 3) split3_bf16x2(x, y, pw[0][i], pw[1][i], pw[2][i]);
                         else split_bf16x2(x, y, pw[0][i], pw[1][i]);
                     }
 #pragma unroll
@@ -645,15 +609,60 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
                         pf[pp][qt][s2] =
                             __builtin_bit_cast(bf16x8_t, make_uint4(pw[pp][0], pw[pp][1], pw[pp][2], pw[pp][3]));
                 }
-                if constexpr (PAIR) ps *= vinv;
                 lsum[qt] += ps;
+            }
+        };
+        auto weigh = [&](int c, bf16x8_t (&pf)[NPP][NQT][NS / 2]) {
+            if constexpr (PLANES) {
+                // as for the scores: the next 32 dims of V during these
+                bf16x8_t vf[2][2][NP];
+                auto load = [&](int d2, bf16x8_t (&f)[2][NP]) {
+#pragma unroll
+                    for (int p = 0; p < NP; ++p)
+#pragma unroll
+                        for (int d = 0; d < 2; ++d) {
+                            const int row = c + lg * 4 + (lq >> 2);
+                            const int off = (p * KT + row) * (kD * 2) +
+                                            ((((2 * d2 + d) * 2 + ((lq & 3) >> 1)) ^ (row & 15)) << 4) + ((lq & 1) << 3);
+                            const v4i16_t lo = lds_read_tr16(vst + off), hi = lds_read_tr16(vst + off + 16 * (kD * 2));
+                            const v8i16_t w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                            f[d][p] = __builtin_bit_cast(bf16x8_t, w);
+                        }
+                };
+                load(0, vf[0]);
+#pragma unroll
+                for (int d2 = 0; d2 < 4; ++d2) {
+                    if (d2 < 3) load(d2 + 1, vf[(d2 + 1) & 1]);
+#pragma unroll
+                    for (int pv = 0; pv < NP; ++pv)
+#pragma unroll
+                        for (int pp = 0; pp < NPP; ++pp) {
+                            if (pv + pp > ORD) continue;
+#pragma unroll
+                            for (int d = 0; d < 2; ++d)
+#pragma unroll
+                                for (int qt = 0; qt < NQT; ++qt)
+                                    o[qt][2 * d2 + d] = mfma16(vf[d2 & 1][d][pv], pf[pp][qt][0], o[qt][2 * d2 + d]);
+                        }
+                }
+                __builtin_amdgcn_sched_group_barrier(0x100, 4 * NP, 0);
+#pragma unroll
+                for (int d2 = 0; d2 < 3; ++d2) {
+#pragma unroll
+                    for (int i = 0; i < 2 * NP; ++i) {
+                        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_group_barrier(0x008, 12, 0);
+                return;
             }
 #pragma unroll
             for (int dt = 0; dt < 8; ++dt) {
 #pragma unroll
                 for (int s2 = 0; s2 < NS / 2; ++s2)
 #pragma unroll
-                    for (int pv_ = 0; pv_ < NP; ++pv_) {     // V plane: hi (then mid and lo, PAIR: lo)
+                    for (int pv_ = 0; pv_ < NP; ++pv_) {     // V plane: hi (then, fp32 V, mid and lo)
                         bf16x8_t va;
                         if constexpr (DMA) {
                             // transposed reads of the row-major tile: lane lq of group lg addresses key
@@ -675,7 +684,7 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
                         for (int pp = 0; pp < NPP; ++pp) {
                             if (pv_ + pp > ORD) continue;     // as for the scores
 #pragma unroll
-                            for (int qt = 0; qt < NQT; ++qt) o[qt][dt] = mfma16<PAIR>(va, pf[pp][qt][s2], o[qt][dt]);
+                            for (int qt = 0; qt < NQT; ++qt) o[qt][dt] = mfma16(va, pf[pp][qt][s2], o[qt][dt]);
                         }
                     }
             }
@@ -683,8 +692,10 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_kernel(PrefillArgs
         for (int c = 0; c < KT && j0 + c < n; c += CH) {
             if (causal && j0 + c > cbase + tw + 16 * NQT - 1) break;   // wave-uniform: the wave's future
             f32x4_t sc[NQT][NS];
+            bf16x8_t pf[NPP][NQT][NS / 2];
             scores(c, sc);
-            finish(c, sc);
+            softmax(c, sc, pf);
+            weigh(c, pf);
         }
         r = rn;
         j0 = jn;
@@ -818,17 +829,18 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_merge_kernel(Prefi
 constexpr int kPrefillNarrowBelow = 256;
 constexpr int kSplitNarrowBelow = 40;
 // Fewer keys than this in every block: the conversion's own launch costs more than the faster tiles give, and fp32
-// K / V are read in place.  12 / 2 heads, causal, in place | planes, us: 64 keys 14.5 | 18.1, 128 20.1 | 17.8, 200
-// 29.5 | 21.8, 512 60.1 | 35.8.
-constexpr int kPairMinKeys = 128;
-enum { kKvBf16 = 0, kKvF32 = 1, kKvPair = 2 };   // bf16, fp32 in place (three bf16 planes), fp32 as fp16 pair planes
+// K / V are split by every workgroup.  Causal, that | planes, us: 100 keys 19.9 | -, 128 20.7 | 18.6, 200 30.2 | 23.7,
+// 512 61.9 | 42.8 at 12 / 2 heads; 128 keys at 4 / 4, 8 / 2, 16 / 2 heads 27.3 | 18.4, 19.2 | 17.4, 21.4 | 19.8.
+constexpr int kPlaneMinKeys = 128;
+constexpr int64_t kPlaneMaxBytes = (int64_t)1 << 37;             // 32-bit workgroup and row counts
+enum { kKvBf16 = 0, kKvF32 = 1, kKvPlanes = 2 };   // bf16, fp32 split by every workgroup, fp32 as planes
 constexpr int prefill_nqt(int grp, int kv) { return kv == kKvBf16 && grp == 8 ? 2 : 1; }
 constexpr int prefill_qw(int grp, int kv, bool narrow) {
     if (kv == kKvF32) return !narrow && (grp == 2 || grp == 4 || grp == 6) ? 2 : 1;
     return (grp == 1 ? 8 : grp == 2 ? 4 : grp == 8 ? 1 : 2) / (narrow && grp != 8 ? 2 : 1);
 }
 // keys per LDS tile
-constexpr int prefill_kt(int kv) { return kv == kKvBf16 ? 128 : kv == kKvPair ? kPairKeys : 32; }
+constexpr int prefill_kt(int kv) { return kv == kKvBf16 ? 128 : 32; }
 
 // Key-range splits: with a workspace, a launch of fewer than kPrefillNarrowBelow workgroups (a
 // 1024-query chunk of the chunk-recurrent prefill at 2 KV heads: 128) splits each tile's keys into up to
@@ -840,15 +852,15 @@ inline int64_t prefill_ws_bytes(int grp) {
     return (int64_t)kPrefillNarrowBelow * prefill_slot_floats(std::max(2 * grp, 4), 2) * 4;
 }
 
-// Launch shape of a call and, for fp32 K / V, the runs that kv_pair_kernel converts (runs over the same rows, as
+// Launch shape of a call and, for fp32 K / V, the runs that kv_planes_kernel converts (runs over the same rows, as
 // two chunks share one, only once).
 struct PrefillPlan {
     int kv = kKvBf16;
     bool narrow = false;
-    int qtile = 0, n_split = 1, split_wgs = 0;
+    int qtile = 0, n_split = 1, plane_wgs = 0;
     int64_t tiles = 0, bytes = 0, max_keys = 0;
-    PairArgs pair{};
-    int run_of[kMaxBlocks][4] = {};        // PAIR: block, run -> pair.run
+    PlaneArgs planes{};
+    int run_of[kMaxBlocks][4] = {};        // planes: block, run -> planes.run
 };
 
 PrefillPlan prefill_plan(int kv, const vgx_attn_block *blocks, int n_blocks, int64_t G, int grp, bool split) {
@@ -866,8 +878,8 @@ PrefillPlan prefill_plan(int kv, const vgx_attn_block *blocks, int n_blocks, int
     p.tiles = count(p.qtile);
     if (split && p.tiles > 0 && p.tiles < kPrefillNarrowBelow)
         p.n_split = (int)std::min<int64_t>(kPrefillMaxSplit, kPrefillNarrowBelow / p.tiles);
-    if (kv != kKvPair) return p;
-    PairArgs &pa = p.pair;
+    if (kv != kKvPlanes) return p;
+    PlaneArgs &pa = p.planes;
     pa.G = (int)G;
     for (int i = 0; i < n_blocks; ++i) {
         int64_t keys = 0;
@@ -879,7 +891,7 @@ PrefillPlan prefill_plan(int kv, const vgx_attn_block *blocks, int n_blocks, int
                                      pa.run[u].gstride != R.group_stride))
                 ++u;
             if (u == pa.n_runs) {
-                PairRun &n = pa.run[pa.n_runs++];
+                PlaneRun &n = pa.run[pa.n_runs++];
                 n.k = static_cast<const float *>(R.k);
                 n.v = static_cast<const float *>(R.v);
                 n.rstride = R.row_stride;
@@ -891,14 +903,11 @@ PrefillPlan prefill_plan(int kv, const vgx_attn_block *blocks, int n_blocks, int
         p.max_keys = std::max(p.max_keys, keys);
     }
     for (int u = 0; u < pa.n_runs; ++u) {
-        PairRun &n = pa.run[u];
-        n.rows = (n.len + kPairKeys - 1) / kPairKeys * kPairKeys;
+        PlaneRun &n = pa.run[u];
         n.planes = reinterpret_cast<uint16_t *>(p.bytes);        // offsets; the call adds the workspace
-        p.bytes += 4 * G * n.rows * kD * 2;
-        n.scale = reinterpret_cast<PairScale *>(p.bytes);
-        p.bytes += (G * (n.rows / kPairKeys) * (int64_t)sizeof(PairScale) + 255) / 256 * 256;
-        n.wg0 = p.split_wgs;
-        p.split_wgs += (int)(n.rows / kPairKeys * G * 2);
+        p.bytes += 6 * G * n.len * kD * 2;                        // (a multiple of 256)
+        n.wg0 = p.plane_wgs;
+        p.plane_wgs += (int)((n.len + kPlaneRows - 1) / kPlaneRows * G * 2);
     }
     return p;
 }
@@ -990,11 +999,10 @@ int attn_prefill_impl(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_b
         if (small) return workspace_bytes < prefill_ws_bytes(grp) ? VGX_E_ARENA : VGX_E_ALIGN;
         p.n_split = 1;
     }
-    // fp32 K / V through the pair planes when the workspace holds them
+    // fp32 K / V through the planes when the workspace holds them
     if (kv_dtype == VGX_F32 && ws_ok && !split) {
-        const PrefillPlan pp = prefill_plan(kKvPair, blocks, n_blocks, G, grp, false);
-        if (pp.bytes <= workspace_bytes && pp.bytes < ((int64_t)1 << 37) && pp.max_keys >= kPairMinKeys)
-            p = pp;                                               // (32-bit workgroup and row counts)
+        const PrefillPlan pp = prefill_plan(kKvPlanes, blocks, n_blocks, G, grp, false);
+        if (pp.bytes <= workspace_bytes && pp.bytes < kPlaneMaxBytes && pp.max_keys >= kPlaneMinKeys) p = pp;
     }
     int64_t tiles = 0;
     for (int i = 0; i < nb; ++i) {
@@ -1005,21 +1013,20 @@ int attn_prefill_impl(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_b
     a.n_tiles = (int)tiles;
     a.n_split = p.n_split;
     a.ws = static_cast<float *>(workspace);
-    if (p.kv == kKvPair) {
+    if (p.kv == kKvPlanes) {
         char *const ws = static_cast<char *>(workspace);
-        for (int u = 0; u < p.pair.n_runs; ++u) {
-            PairRun &n = p.pair.run[u];
+        for (int u = 0; u < p.planes.n_runs; ++u) {
+            PlaneRun &n = p.planes.run[u];
             n.planes = reinterpret_cast<uint16_t *>(ws + reinterpret_cast<int64_t>(n.planes));
-            n.scale = reinterpret_cast<PairScale *>(ws + reinterpret_cast<int64_t>(n.scale));
         }
         for (int i = 0; i < nb; ++i)
             for (int r = 0; r < a.blk[i].n_runs; ++r) {
-                const PairRun &n = p.pair.run[p.run_of[a.blk[i].src][r]];
+                const PlaneRun &n = p.planes.run[p.run_of[a.blk[i].src][r]];
                 a.blk[i].run[r].k = n.planes;
-                a.blk[i].run[r].v = n.scale;
-                a.blk[i].run[r].rstride = n.rows;
+                a.blk[i].run[r].v = nullptr;
+                a.blk[i].run[r].rstride = n.len;
             }
-        hipLaunchKernelGGL(kv_pair_kernel, dim3((unsigned)p.split_wgs), dim3(256), 0, (hipStream_t)stream, p.pair);
+        hipLaunchKernelGGL(kv_planes_kernel, dim3((unsigned)p.plane_wgs), dim3(256), 0, (hipStream_t)stream, p.planes);
         VGX_CHECK_LAUNCH();
     }
     const bool narrow = p.narrow;
@@ -1038,8 +1045,8 @@ int attn_prefill_impl(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_b
     if (narrow) VGX_PREFILL_SHAPE(G_, S_, KV_, true); else VGX_PREFILL_SHAPE(G_, S_, KV_, false)
 #define VGX_PREFILL_GO(G_, S_)                                     \
     do {                                                           \
-        if (p.kv == kKvPair) {                                     \
-            VGX_PREFILL_KV(G_, S_, kKvPair);                       \
+        if (p.kv == kKvPlanes) {                                     \
+            VGX_PREFILL_KV(G_, S_, kKvPlanes);                       \
         } else if (p.kv == kKvF32) {                               \
             VGX_PREFILL_KV(G_, S_, kKvF32);                        \
         } else {                                                   \
@@ -1095,8 +1102,8 @@ int64_t vgx_attn_prefill_planes_bytes(int kv_dtype, const vgx_attn_block *blocks
         for (int r = 0; r < blocks[i].n_runs; ++r)
             if (blocks[i].runs[r].len < 0) return VGX_E_SIZE;
     }
-    const PrefillPlan p = prefill_plan(kKvPair, blocks, n_blocks, G, grp, false);
-    return p.max_keys >= kPairMinKeys ? p.bytes : 0;
+    const PrefillPlan p = prefill_plan(kKvPlanes, blocks, n_blocks, G, grp, false);
+    return p.max_keys >= kPlaneMinKeys && p.bytes < kPlaneMaxBytes ? p.bytes : 0;
 }
 
 int vgx_attn_prefill_ws(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_block *blocks, int n_blocks, int64_t H,

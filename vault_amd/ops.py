@@ -549,8 +549,7 @@ def attn_prefill(blocks, H: int, G: int, scale: Optional[float] = None, ws: Opti
 
     Each block is a dict: ``q`` [n_q, H, D] view (fp32 or bf16, any token / head stride, D contiguous),
     ``out`` [n_q, H, D] view, fp32 or bf16 (one dtype for all blocks), ``runs``: list of (K, V) views
-    [G, n, D] (bf16, or fp32 entering the MFMAs in 16-bit pieces that hold 22 bits or more; one dtype
-    for all runs; D contiguous, any row and group stride), ``causal_base``: -1, or b >= 0 making the last run causal (query t sees
+    [G, n, D] (bf16, or fp32 entering the MFMAs as three bf16 pieces; one dtype for all runs; D contiguous, any row and group stride), ``causal_base``: -1, or b >= 0 making the last run causal (query t sees
     its keys j <= b + t).  Optional ``bias`` fp32 [n_q, R, >= run length] with ``bias_head_row`` (H
     ints: the bias row of head h, < 0: none) and ``bias_run``: query t of head h adds
     bias[t, bias_head_row[h], j] to its score with key j of that run.  With ``ws`` (a Workspace) a launch
@@ -570,7 +569,7 @@ def attn_prefill(blocks, H: int, G: int, scale: Optional[float] = None, ws: Opti
     for i0 in range(0, len(blocks), 8):
         part = blocks[i0:i0 + 8]
         arr = (L.AttnBlock * len(part))()
-        keep = []
+        keep, max_keys = [], 0
         for i, b in enumerate(part):
             q, out = b["q"], b["out"]
             if q.dtype != qdt or out.dtype != odt or q.stride(-1) != 1 or out.stride(-1) != 1:
@@ -578,14 +577,17 @@ def attn_prefill(blocks, H: int, G: int, scale: Optional[float] = None, ws: Opti
             runs = b["runs"]
             if not 1 <= len(runs) <= 4:
                 raise ValueError("1 to 4 key runs per block")
-            ra = (L.KVRun * 4)()
+            ra, keys = (L.KVRun * 4)(), 0
             for j, (k, v) in enumerate(runs):
                 if k.dtype != kvdt or v.dtype != kvdt or k.shape != v.shape:
                     raise ValueError("key runs must be K/V of one dtype and shape")
                 if k.stride(-1) != 1 or v.stride(-1) != 1 or k.stride(0) != v.stride(0) or k.stride(1) != v.stride(1):
                     raise ValueError("K and V views need equal strides and contiguous rows")
-                ra[j] = L.KVRun(k.data_ptr(), v.data_ptr(), k.shape[1], k.stride(1), k.stride(0))
+                n = k.shape[1]
+                ra[j] = L.KVRun(k.data_ptr(), v.data_ptr(), n, k.stride(1), k.stride(0))
                 keep.append((k, v))
+                keys += n
+            max_keys = max(max_keys, keys)
             arr[i] = L.AttnBlock(q.data_ptr(), q.stride(0), q.stride(1), out.data_ptr(), out.stride(0), out.stride(1),
                                  q.shape[0], int(b.get("causal_base", -1)), len(runs), ra)
             if b.get("bias") is not None:
@@ -603,31 +605,33 @@ def attn_prefill(blocks, H: int, G: int, scale: Optional[float] = None, ws: Opti
                 keep.append((bias, rows_dev))
         qd = L.BF16 if qdt == torch.bfloat16 else L.F32
         od = L.BF16 if odt == torch.bfloat16 else L.F32
-        _prefill_launch(C.addressof(arr), len(part), kvdt, qd, od, H, G, D, scale, ws, part[0]["q"].device)
+        _prefill_launch(C.addressof(arr), len(part), kvdt, qd, od, H, G, D, scale, ws, part[0]["q"].device, max_keys)
 
 
 # vgx_attn_block as 64-bit words (its two ints are padded to 8 bytes): q, ldq, q_hstride, out, ldo, o_hstride, n_q,
 # causal_base, n_runs, four runs of (k, v, len, row_stride, group_stride), bias, bias_head_row, bias_ldq,
 # bias_rstride, bias_run
 PREFILL_BLOCK_WORDS = 34
+# blocks of fewer keys never take the planes (kPlaneMinKeys): spares them the call that asks for their size
+PLANE_MIN_KEYS = 128
 assert C.sizeof(L.AttnBlock) == 8 * PREFILL_BLOCK_WORDS and sys.byteorder == "little"
 
 
 def attn_prefill_words(words: list, kvdt: torch.dtype, qdt: torch.dtype, odt: torch.dtype, H: int, G: int,
-                       D: int, scale: float, dev: torch.device) -> None:
-    """attn_prefill over blocks given as PREFILL_BLOCK_WORDS words each, for callers whose blocks are
-    regular: filling them from tensor views costs the host about 20 us a block, a list of words 3."""
+                       D: int, scale: float, dev: torch.device, max_keys: int) -> None:
+    """attn_prefill over blocks given as PREFILL_BLOCK_WORDS words each, none of more than max_keys keys, for callers
+    whose blocks are regular: filling them from tensor views costs the host about 20 us a block, a list of words 3."""
     arr = (C.c_int64 * len(words))(*words)
     n = len(words) // PREFILL_BLOCK_WORDS
     qd = L.BF16 if qdt == torch.bfloat16 else L.F32
     od = L.BF16 if odt == torch.bfloat16 else L.F32
     for i0 in range(0, n, 8):
         _prefill_launch(C.addressof(arr) + 8 * PREFILL_BLOCK_WORDS * i0, min(8, n - i0), kvdt, qd, od, H, G, D, scale,
-                        None, dev)
+                        None, dev, max_keys)
 
 
 def _prefill_launch(blocks: int, n: int, kvdt: torch.dtype, qd: int, od: int, H: int, G: int, D: int, scale: float,
-                    ws: Optional["Workspace"], dev: torch.device) -> None:
+                    ws: Optional["Workspace"], dev: torch.device, max_keys: int) -> None:
     lib = L.load()
     kd = KV_DTYPES[kvdt]
     need = 0
@@ -638,12 +642,17 @@ def _prefill_launch(blocks: int, n: int, kvdt: torch.dtype, qd: int, od: int, H:
         L.check(lib.vgx_attn_prefill_ws(kd, qd, od, blocks, n, H, G, D, scale, buf.data_ptr(), buf.numel(), _stream(dev)),
                 "vgx_attn_prefill_ws")
         return
-    if kvdt == torch.float32 and D == 128:
+    if kvdt == torch.float32 and D == 128 and max_keys >= PLANE_MIN_KEYS:
         need = int(lib.vgx_attn_prefill_planes_bytes(kd, blocks, n, H, G))
         L.check(min(need, 0), "vgx_attn_prefill_planes_bytes")
+    buf = None
     if need:
-        # scratch of this call (stream-ordered) for the fp16 planes of K / V
-        buf = torch.empty(need, dtype=torch.uint8, device=dev)
+        # scratch of this call (stream-ordered) for the planes of K / V; without room for them, the same bits more slowly
+        try:
+            buf = torch.empty(need, dtype=torch.uint8, device=dev)
+        except torch.OutOfMemoryError:
+            pass
+    if buf is not None:
         L.check(lib.vgx_attn_prefill_planes(kd, qd, od, blocks, n, H, G, D, scale, buf.data_ptr(), need, _stream(dev)),
                 "vgx_attn_prefill_planes")
     else:
