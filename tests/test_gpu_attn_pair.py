@@ -181,3 +181,26 @@ def test_prefill_zero_values_keep_their_weight(dev, big):
     out = torch.empty(T, H, 128, device=dev)
     ops.attn_prefill([{"q": q, "out": out, "runs": runs, "causal_base": 0}], H, G)
     assert np.abs(out.double().cpu().numpy() - _ref(q, runs)).max() <= TOL32 * big
+
+
+@pytest.mark.parametrize("kvdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [100, 1024])
+def test_prefill_workspace_sizes_one_head_per_group(dev, kvdt, T):
+    """One head per group: the workspace of vgx_attn_prefill_workspace_bytes and half of it serve the call, less is
+    refused (a launch of 256 workgroups or more runs unsplit)."""
+    rng, lib, H = np.random.default_rng(T), L.load(), 8
+    runs = [tuple(_t(rng.standard_normal((H, n, 128)), kvdt) for _ in range(2)) for n in (77, T)]
+    q, out = _t(rng.standard_normal((T, H, 128))), torch.empty(T, H, 128, device=dev)
+    ref = _ref(q, runs)
+    ra = (L.KVRun * 4)(*[L.KVRun(k.data_ptr(), v.data_ptr(), k.shape[1], k.stride(1), k.stride(0)) for k, v in runs])
+    arr = (L.AttnBlock * 1)(L.AttnBlock(q.data_ptr(), q.stride(0), q.stride(1), out.data_ptr(), out.stride(0),
+                                        out.stride(1), T, 0, 2, ra))
+    full = int(lib.vgx_attn_prefill_workspace_bytes(H, H))
+    for size in (full, full // 2, full // 2 - 1):
+        ws = torch.full((size + 4096,), 7, dtype=torch.uint8, device=dev)
+        out.fill_(7.0)
+        rc = lib.vgx_attn_prefill_ws(L.BF16 if kvdt == torch.bfloat16 else L.F32, L.F32, L.F32, arr, 1, H, H, 128, 128 ** -0.5,
+                                     ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream)
+        assert (rc == 0) == (size >= full // 2 or T == 1024) and int((ws[size:] != 7).sum()) == 0
+        if rc == 0:
+            assert np.abs(out.double().cpu().numpy() - ref).max() <= (TOL32 if kvdt == torch.float32 else TOL)

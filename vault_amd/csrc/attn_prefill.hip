@@ -847,9 +847,10 @@ constexpr int prefill_kt(int kv) { return kv == kKvBf16 ? 128 : 32; }
 // four ranges, so that the launch fills the CUs; attn_prefill_merge_kernel then combines them.
 
 // Workspace bound: at most kPrefillNarrowBelow (tile, range) slots, each of at most 2 GRP waves x 2
-// 16-query tiles (one head per group: 8 waves of one).
-inline int64_t prefill_ws_bytes(int grp) {
-    return (int64_t)kPrefillNarrowBelow * prefill_slot_floats(std::max(2 * grp, 4), 2) * 4;
+// 16-query tiles (one head per group: 8 waves of one, half of that for its narrow shape, which a workspace
+// of that size gets).
+inline int64_t prefill_ws_bytes(int grp, bool narrow = false) {
+    return (int64_t)kPrefillNarrowBelow * prefill_slot_floats(grp == 1 && !narrow ? 4 : 2 * grp, 2) * 4;
 }
 
 // Launch shape of a call and, for fp32 K / V, the runs that kv_planes_kernel converts (runs over the same rows, as
@@ -863,7 +864,8 @@ struct PrefillPlan {
     int run_of[kMaxBlocks][4] = {};        // planes: block, run -> planes.run
 };
 
-PrefillPlan prefill_plan(int kv, const vgx_attn_block *blocks, int n_blocks, int64_t G, int grp, bool split) {
+// may_wide: whether key ranges may take the wide shape (the workspace holds its slots).
+PrefillPlan prefill_plan(int kv, const vgx_attn_block *blocks, int n_blocks, int64_t G, int grp, bool split, bool may_wide) {
     PrefillPlan p;
     p.kv = kv;
     auto count = [&](int q) {
@@ -873,7 +875,8 @@ PrefillPlan prefill_plan(int kv, const vgx_attn_block *blocks, int n_blocks, int
         return t;
     };
     const int wide = kv == kKvF32 ? 32 : 16 * prefill_nqt(grp, kv) * prefill_qw(grp, kv, false);
-    p.narrow = prefill_qw(grp, kv, false) > 1 && count(wide) < (split && kv != kKvF32 ? kSplitNarrowBelow : kPrefillNarrowBelow);
+    p.narrow = prefill_qw(grp, kv, false) > 1 &&
+               count(wide) < (split && may_wide && kv != kKvF32 ? kSplitNarrowBelow : kPrefillNarrowBelow);
     p.qtile = 16 * prefill_nqt(grp, kv) * prefill_qw(grp, kv, p.narrow);   // queries per workgroup
     p.tiles = count(p.qtile);
     if (split && p.tiles > 0 && p.tiles < kPrefillNarrowBelow)
@@ -984,10 +987,11 @@ int attn_prefill_impl(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_b
         ++nb;
     }
     if (nb == 0) return VGX_OK;
-    PrefillPlan p = prefill_plan(kv_dtype == VGX_F32 ? kKvF32 : kKvBf16, blocks, n_blocks, G, grp, split);
+    PrefillPlan p = prefill_plan(kv_dtype == VGX_F32 ? kKvF32 : kKvBf16, blocks, n_blocks, G, grp, split,
+                                 workspace_bytes >= prefill_ws_bytes(grp));
     if (p.tiles > 0x7FFFFFFF) return VGX_E_LIMIT;
     const bool ws_ok = workspace && (uintptr_t)workspace % 16 == 0;
-    if (split && !(ws_ok && workspace_bytes >= prefill_ws_bytes(grp))) {
+    if (split && !(ws_ok && workspace_bytes >= prefill_ws_bytes(grp, true))) {
         // refused for a launch of few 32-query tiles (16-query ones where two waves share a head), else unsplit
         int64_t t32 = 0, t16 = 0;
         for (int i = 0; i < nb; ++i) {
@@ -996,12 +1000,12 @@ int attn_prefill_impl(int kv_dtype, int q_dtype, int out_dtype, const vgx_attn_b
         }
         const bool small = kv_dtype == VGX_F32 ? p.tiles < kPrefillNarrowBelow
                                                : (grp == 4 || grp == 6 ? t16 : t32) < kPrefillNarrowBelow;
-        if (small) return workspace_bytes < prefill_ws_bytes(grp) ? VGX_E_ARENA : VGX_E_ALIGN;
+        if (small) return workspace_bytes < prefill_ws_bytes(grp, true) ? VGX_E_ARENA : VGX_E_ALIGN;
         p.n_split = 1;
     }
     // fp32 K / V through the planes when the workspace holds them
     if (kv_dtype == VGX_F32 && ws_ok && !split) {
-        const PrefillPlan pp = prefill_plan(kKvPlanes, blocks, n_blocks, G, grp, false);
+        const PrefillPlan pp = prefill_plan(kKvPlanes, blocks, n_blocks, G, grp, false, false);
         if (pp.bytes <= workspace_bytes && pp.bytes < kPlaneMaxBytes && pp.max_keys >= kPlaneMinKeys) p = pp;
     }
     int64_t tiles = 0;
@@ -1102,7 +1106,7 @@ int64_t vgx_attn_prefill_planes_bytes(int kv_dtype, const vgx_attn_block *blocks
         for (int r = 0; r < blocks[i].n_runs; ++r)
             if (blocks[i].runs[r].len < 0) return VGX_E_SIZE;
     }
-    const PrefillPlan p = prefill_plan(kKvPlanes, blocks, n_blocks, G, grp, false);
+    const PrefillPlan p = prefill_plan(kKvPlanes, blocks, n_blocks, G, grp, false, false);
     return p.max_keys >= kPlaneMinKeys && p.bytes < kPlaneMaxBytes ? p.bytes : 0;
 }
 
