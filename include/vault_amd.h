@@ -140,6 +140,11 @@ int vgx_qlinear_indirect(int dtype, const void *w_packed, int64_t rows, int64_t 
  * same workspace may serve vgx_qkv_rope_batch, which leaves the counter region untouched. */
 int64_t vgx_qgemm_workspace_bytes(int64_t batch, int64_t rows, int64_t cols, int epilogue);
 
+/* The same for weights of one dtype (vgx_qgemm_workspace_bytes serves every dtype): VGX_Q8_0 and VGX_Q4_0 without the
+ * third activation plane of the 16-bit types, those without the needs of the quantized ones; 0 where the call takes
+ * no workspace. */
+int64_t vgx_qgemm_workspace_bytes_of(int dtype, int64_t batch, int64_t rows, int64_t cols, int epilogue);
+
 /* vgx_qlinear_ex for many activation rows on bf16 MFMA (Q8_0 / Q4_0 weights): same arguments and
  * epilogues, plus a caller workspace.  The activations (after the optional RMSNorm) enter as a bf16
  * hi + lo pair (2^-17 relative); weights, scales and the per-block fp32 accumulation are exact as in

@@ -53,6 +53,21 @@ def test_host_validation_codes(lib):
     assert lib.vgx_qlinear(L.Q4_0, p, 4, 32, p, 32, 0, None, p, 4, 0, None) == 0   # empty batch: no-op
 
 
+@pytest.mark.parametrize("batch,rows,cols,epi", [(1, 64, 64, 0), (16, 1536, 8960, 1), (40, 8960, 1536, 2), (333, 1536, 8960, 1),
+                                                 (1024, 8960, 1536, 2), (16, 151665, 1536, 0), (9, 64, 64, 0)])
+def test_qgemm_workspace_of_a_dtype(lib, batch, rows, cols, epi):
+    """The workspace of one dtype is within the one for all; quantized weights hold two activation planes, 16-bit ones
+    three or nothing, F32 nothing."""
+    every = lib.vgx_qgemm_workspace_bytes(batch, rows, cols, epi)
+    of = {dt: lib.vgx_qgemm_workspace_bytes_of(dt, batch, rows, cols, epi) for dt in (L.Q4_0, L.Q8_0, L.F32, L.BF16, L.F16)}
+    plane = (batch * cols * 2 + 255) // 256 * 256
+    assert every == max(of.values()) and of[L.F32] == 0 and of[L.Q4_0] == of[L.Q8_0] >= 65536 + 2 * plane
+    for dt in (L.BF16, L.F16):
+        assert of[dt] >= 65536 + 3 * plane if cols >= 768 else of[dt] == 0
+    assert lib.vgx_qgemm_workspace_bytes_of(3, batch, rows, cols, epi) == -5
+    assert lib.vgx_qgemm_workspace_bytes_of(L.Q4_0, batch, rows, 33, epi) == -7
+
+
 def test_state_has_no_reference_cycle():
     """A decode state must be freed by reference counting alone: a state left to the cyclic garbage
     collector can be collected while a decode graph is being captured, and its destructors (pinned

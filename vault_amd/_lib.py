@@ -50,6 +50,7 @@ _SIGS = {
     "vgx_qlinear_indirect": (I32, [I32, P, I64, I64, P, I64, I64, P, F, P, P, I64, I32, P]),
     "vgx_qlinear_side": (I32, [I32, P, I64, I64, P, I64, I64, P, F, P, P, I64, I32, P, P]),
     "vgx_qgemm_workspace_bytes": (I64, [I64, I64, I64, I32]),
+    "vgx_qgemm_workspace_bytes_of": (I64, [I32, I64, I64, I64, I32]),
     "vgx_qgemm": (I32, [I32, P, I64, I64, P, I64, I64, P, F, P, P, I64, I32, P, I64, P]),
     "vgx_attn_decode_workspace_bytes": (I64, [I64, I64, I64, I64, I64]),
     "vgx_attn_decode": (I32, [I32, P, I64, P, I32, P, I64, I32, I64, P, I64, I64, I64, I64, F, P, I64, P]),

@@ -2427,6 +2427,12 @@ inline int64_t wgemm_bytes(int64_t batch, int64_t n_rq, int nblk) {
            part_bytes(wgemm_ksplit(n_rq, batch, nblk), batch, n_rq * 4);
 }
 
+// Whether the weights and the planes lie within the DMA's buffer ranges.
+inline bool wgemm_fits(int64_t batch, int64_t n_rq, int nblk) {
+    return n_rq * nblk * 256 < ((int64_t)1 << 31) &&
+           kPlanes * split_plane_bytes(batch, (int64_t)nblk * QK) < ((int64_t)1 << 31);
+}
+
 // Whether wgemm_tile_kernel is ahead of f32gemm_tile_kernel for `tiles` 64 x 64 tiles of the latter.  Below 16 blocks
 // (no K splits) it waits out its pre-pass and one K range on few CUs, while the fp32 kernel is done after one round
 // of its tiles over the CUs.  Times fp32 | this, us, BF16 (F16): 64 columns 256 tiles 6.6 | 13, 512 tiles at 0.72
@@ -2478,18 +2484,34 @@ int wgemm_launch(const void *w_packed, int64_t rows, int64_t n_rq, int nblk, con
 
 extern "C" {
 
-int64_t vgx_qgemm_workspace_bytes(int64_t batch, int64_t rows, int64_t cols, int epilogue) {
+int64_t vgx_qgemm_workspace_bytes_of(int dtype, int64_t batch, int64_t rows, int64_t cols, int epilogue) {
+    if (dtype != VGX_Q8_0 && dtype != VGX_Q4_0 && dtype != VGX_F32 && dtype != VGX_BF16 && dtype != VGX_F16)
+        return VGX_E_DTYPE;
     if (batch <= 0 || rows <= 0 || cols <= 0) return VGX_E_SIZE;
     if (cols % QK) return VGX_E_SHAPE;
+    if (dtype == VGX_F32) return 0;
     const int64_t rows_p = rows4(epilogue == VGX_EPI_SWIGLU ? 2 * rows : rows);
-    const int ks = tile_ksplit(rows_p / 4, batch, (int)(cols / QK));
+    const int nblk = (int)(cols / QK);
+    if (dtype == VGX_BF16 || dtype == VGX_F16) {
+        const bool pays = wgemm_pays(dtype, nblk, (rows_p + kFT - 1) / kFT * ((batch + kFT - 1) / kFT), batch);
+        return pays && wgemm_fits(batch, rows_p / 4, nblk) ? wgemm_bytes(batch, rows_p / 4, nblk) : 0;
+    }
+    const int ks = tile_ksplit(rows_p / 4, batch, nblk);
     const int64_t big = kQgemmTicketBytes + split_bytes(batch, cols) + part_bytes(ks, batch, rows_p);
-    // the weight dtype is not an argument: the larger of the Q4_0 and Q8_0 layouts
-    const int64_t sq4 = small_bytes(batch, rows_p / 4, (int)(cols / QK), VGX_Q4_0);
-    const int64_t sq8 = small_bytes(batch, rows_p / 4, (int)(cols / QK), VGX_Q8_0);
-    // ... nor is it for the BF16 / F16 layout
-    const int64_t all = std::max(big, wgemm_bytes(batch, rows_p / 4, (int)(cols / QK)));
-    return batch <= kSmallMaxBatch ? std::max(all, std::max(sq4, sq8)) : all;
+    // Q4_0 and Q8_0 alike: a workspace for one serves the other
+    const int64_t sq4 = small_bytes(batch, rows_p / 4, nblk, VGX_Q4_0);
+    const int64_t sq8 = small_bytes(batch, rows_p / 4, nblk, VGX_Q8_0);
+    return batch <= kSmallMaxBatch ? std::max(big, std::max(sq4, sq8)) : big;
+}
+
+int64_t vgx_qgemm_workspace_bytes(int64_t batch, int64_t rows, int64_t cols, int epilogue) {
+    int64_t need = 0;
+    for (int dt : {VGX_Q4_0, VGX_BF16, VGX_F16}) {
+        const int64_t n = vgx_qgemm_workspace_bytes_of(dt, batch, rows, cols, epilogue);
+        if (n < 0) return n;
+        need = std::max(need, n);
+    }
+    return need;
 }
 
 int vgx_qgemm(int dtype, const void *w_packed, int64_t rows, int64_t cols, const float *x, int64_t ldx, int64_t batch,
@@ -2515,11 +2537,9 @@ int vgx_qgemm(int dtype, const void *w_packed, int64_t rows, int64_t cols, const
         // down of BF16 files at 8, 40, 333, 1024 rows: 107 -> 25, 108 -> 33, 243 -> 76, 591 -> 184 us | 472 -> 24,
         // 474 -> 28, 462 -> 53, 467 -> 107 us
         const dim3 grid((unsigned)((n_rq + kFT / 4 - 1) / (kFT / 4)), (unsigned)((batch + kFT - 1) / kFT));
-        const int64_t pbytes = kPlanes * split_plane_bytes(batch, cols);
         if (dtype != VGX_F32 && wgemm_pays(dtype, nblk, (int64_t)grid.x * grid.y, batch) && workspace &&
             (uintptr_t)workspace % 256 == 0 && (uintptr_t)w_packed % 16 == 0 &&
-            workspace_bytes >= wgemm_bytes(batch, n_rq, nblk) && n_rq * nblk * 256 < ((int64_t)1 << 31) &&
-            pbytes < ((int64_t)1 << 31)) {
+            wgemm_fits(batch, n_rq, nblk) && workspace_bytes >= wgemm_bytes(batch, n_rq, nblk)) {
             if (dtype == VGX_BF16)
                 return wgemm_launch<VGX_BF16>(w_packed, rows, n_rq, nblk, x, ldx, batch, bias, y, ldy, epilogue, workspace,
                                               (hipStream_t)stream);

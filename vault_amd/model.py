@@ -687,7 +687,7 @@ class VAULTv3ForCausalLM:
                       ((cfg.n_heads + 2 * cfg.n_kv_heads) * cfg.head_dim, cfg.d_model, ops.L.EPI_STORE),
                       (cfg.d_model, cfg.n_heads * cfg.head_dim, ops.L.EPI_ACCUM),
                       (cfg.vocab_size, cfg.d_model, ops.L.EPI_STORE)]
-            need = max(int(lib.vgx_qgemm_workspace_bytes(st.batch, r, c, e)) for r, c, e in shapes)
+            need = max(int(lib.vgx_qgemm_workspace_bytes_of(ops.Q4_0, st.batch, r, c, e)) for r, c, e in shapes)
             if self._batch_qkv_fusable(st.batch):
                 need = max([need] + [int(lib.vgx_qkv_rope_batch_workspace_bytes(
                     st.batch, cfg.d_model, cfg.n_heads, cfg.n_kv_heads, cfg.head_dim, sep)) for sep in (0, 1)])

@@ -172,19 +172,21 @@ def _gemv(w: QWeight, x: torch.Tensor, out: Optional[torch.Tensor], epi: int, bi
     if nw is not None:
         _need(nw, torch.float32, "norm weight")
     if B >= GEMM_MIN_ROWS and w.dtype in ELEM_BYTES and nw is not None:
-        # plain weights: the fp32 MFMA GEMM has no RMSNorm prologue; normalise first
+        # plain weights: their GEMMs have no RMSNorm prologue; normalise first
         x2 = rmsnorm(x2, nw, eps)
         nw = None
     if B >= GEMM_MIN_ROWS and (w.dtype in (Q8_0, Q4_0) or w.dtype in ELEM_BYTES):
         lib = L.load()
-        need = int(lib.vgx_qgemm_workspace_bytes(B, w.rows, w.cols, epi))
+        need = int(lib.vgx_qgemm_workspace_bytes_of(w.dtype, B, w.rows, w.cols, epi))
         # BF16 / F16 weights take no tickets: scratch of their own per call (stream-ordered), so that calls on
         # several streams stay independent
-        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if w.dtype in (BF16, F16) else \
-            gemm_workspace(x.device).get(need)
+        ws = None
+        if need > 0:
+            ws = torch.empty(need, dtype=torch.uint8, device=x.device) if w.dtype in (BF16, F16) else \
+                gemm_workspace(x.device).get(need)
         L.check(lib.vgx_qgemm(w.dtype, w.packed.data_ptr(), w.rows, w.cols, x2.data_ptr(), x2.stride(0), B, _ptr(nw),
-                              float(eps), _ptr(bias), y2.data_ptr(), y2.stride(0), epi, ws.data_ptr(), ws.numel(),
-                              _stream(x.device)), "vgx_qgemm")
+                              float(eps), _ptr(bias), y2.data_ptr(), y2.stride(0), epi, _ptr(ws),
+                              ws.numel() if ws is not None else 0, _stream(x.device)), "vgx_qgemm")
         return out
     L.check(L.load().vgx_qlinear_ex(w.dtype, w.packed.data_ptr(), w.rows, w.cols, x2.data_ptr(), x2.stride(0), B,
                                     _ptr(nw), float(eps), _ptr(bias), y2.data_ptr(), y2.stride(0), epi,
