@@ -2413,7 +2413,6 @@ int split_proj_launch(int dtype, const void *wp, int64_t rows, int64_t cols, con
 
 // BF16 / F16 weights on wgemm_tile_kernel: planes, K-split partials, past the tile counters
 // (which the next decode batch on the same workspace takes its tickets from).
-constexpr int kWgTM = 256, kWgTN = 64, kWgNS = 2;
 // K splits: as many as fit 512 workgroups (one round at two per CU), at least 8 blocks each.
 inline int wgemm_ksplit(int64_t n_rq, int64_t batch, int nblk) {
     const int64_t tiles = (n_rq + kWgTM / 4 - 1) / (kWgTM / 4) * ((batch + kWgTN - 1) / kWgTN);
@@ -2460,7 +2459,7 @@ int wgemm_launch(const void *w_packed, int64_t rows, int64_t n_rq, int nblk, con
     const dim3 grid((unsigned)((n_rq + kWgTM / 4 - 1) / (kWgTM / 4)), (unsigned)((batch + kWgTN - 1) / kWgTN), (unsigned)ks);
     const auto *w = static_cast<const uint8_t *>(w_packed);
 #define VGX_WG(EPI, SP)                                                                                            \
-    hipLaunchKernelGGL((wgemm_tile_kernel<WDT, EPI, SP, kWgTM, kWgTN, kWgNS>), grid, dim3(kWgTM * kWgTN / 64), 0, st, w, \
+    hipLaunchKernelGGL((wgemm_tile_kernel<WDT, EPI, SP>), grid, dim3(kWgTM), 0, st, w,              \
                        n_rq, nblk, rows, xs, pb / 2, x, ldx, batch, bias, y, ldy, part, kper)
     if (ks > 1) VGX_WG(EPI_STORE, true);
     else if (epilogue == VGX_EPI_SWIGLU) VGX_WG(EPI_SWIGLU, false);

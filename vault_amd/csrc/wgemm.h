@@ -9,16 +9,18 @@
 // (8 + 3 bits, exact over fp16's whole range), widened from the staged tile.  All pieces of a block accumulate
 // into one fp32 accumulator.
 //
-// What bounds it: at chunk sizes the matrix cores at three (two) times the product's operations (gate/up
+// What bounds it: at chunk sizes the matrix cores at three (F16: six) times the product's operations (gate/up
 // 2 x 8960 x 1536 over 1024 rows: 184 us, 306 TFLOP/s of the product, 920 of the pieces, against 1200 of
 // a large library product), below about 100 rows the weights' HBM stream (55 MB, 25 us) and the padding
 // of the 64-row tile.  The fp32 MFMA that f32gemm_tile_kernel runs has 1/16 of the 16-bit rate (gate/up
-// 591 us at 95 TFLOP/s; down 1536 x 8960, 96 workgroups without K splits: 467 us against 107).
+// 591 us at 95 TFLOP/s; down 1536 x 8960, 384 workgroups of 64 x 64 whose chain of 280 blocks is not split: 467
+// us against 107).
 #pragma once
 
 namespace {
 
 constexpr int kPlanes = 3;
+constexpr int kWgTM = 256, kWgTN = 64;     // weight rows x activation rows of a tile
 
 // Three bf16 planes of the activations, natural order: plane p of row b at xs + p * pstride + b * cols.
 // One thread per four elements.
@@ -87,25 +89,22 @@ __device__ float wgemm_plain_dot(const uint8_t *__restrict__ W, int nblk, int64_
     return s;
 }
 
-// Tile of TM weight rows x TN activation rows, a wave 64 x 64 (wave w: weight rows 64 (w % (TM / 64)),
-// activation rows 64 (w / (TM / 64))).  Stages of one 32-wide K block of the weights and of every
-// activation plane are filled by LDS DMA, NS in a ring: the loads of block k + NS - 1 leave behind the
-// barrier of block k.  Every wave issues the same number of loads per block, also past the range (zeros),
-// so that the wait for block k is one constant.  Rows of a stage are 64 bytes (one block), their 16-byte
+// Tile of 256 weight rows x 64 activation rows, a wave 64 x 64.  Two stages of one 32-wide K block of the weights
+// and of every activation plane are filled by LDS DMA: the loads of block k + 1 leave behind the barrier of
+// block k (past the range they read zeros).  Rows of a stage are 64 bytes (one block), their 16-byte
 // pieces swizzled by (row >> 2) & 3 against bank conflicts of the MFMA operand reads.  M0 is written by
 // the DMA alone (checked in the compiled code, as dma16 asks).
 // Tiles measured (BF16, gate/up | down over 333 and 1024 rows, us): 256 x 64 with two stages 76, 184 | 53,
 // 107; 128 x 128 78, 187 | 53, 108; 256 x 64 with three stages (one workgroup per CU) 94, 222 | 58, 115;
 // 256 x 128 of eight waves with two stages 83, 176 | 65, 105, with three 93, 203 | 71, 114.
-template <int WDT, int EPI, bool SPLIT, int TM, int TN, int NS>
-__global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm_tile_kernel(
+template <int WDT, int EPI, bool SPLIT>
+__global__ __launch_bounds__(256, 2) void wgemm_tile_kernel(
     const uint8_t *__restrict__ W, int64_t n_rq, int nblk, int64_t rows_out, const uint16_t *__restrict__ xs,
     int64_t pstride, const float *__restrict__ x, int64_t ldx, int64_t batch, const float *__restrict__ bias,
     float *__restrict__ y, int64_t ldy, float *__restrict__ part, int kper) {
     constexpr int NP = kPlanes;
     constexpr int NW = WDT == VGX_F16 ? 2 : 1;         // bf16 pieces of a weight
-    constexpr int NWAVE = TM / 64 * (TN / 64);
-    constexpr int NT = 64 * NWAVE;
+    constexpr int TM = kWgTM, TN = kWgTN, NWAVE = TM / 64, NT = 64 * NWAVE;
     constexpr int A_B = TM * QK * 2, BH_B = TN * QK * 2;
     constexpr int STAGE_B = A_B + NP * BH_B;
     constexpr int NJ = STAGE_B / 1024;                 // wave-loads per block
@@ -113,12 +112,11 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
     static_assert(NJ % NWAVE == 0, "every wave issues the same loads");
     constexpr int kERow = 64 + 4;
     constexpr int EPI_B = TN * kERow * 4;
-    __shared__ __align__(16) uint8_t smem[NS * STAGE_B > EPI_B ? NS * STAGE_B : EPI_B];
+    __shared__ __align__(16) uint8_t smem[2 * STAGE_B > EPI_B ? 2 * STAGE_B : EPI_B];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, lg = lane >> 4;
-    const int wm = wave % (TM / 64), wn = wave / (TM / 64);
     const int cols = nblk * QK;
     // XCD-aware tile order, as qgemm_tile_dma_kernel's
     int tr = blockIdx.x, tt = blockIdx.y;
@@ -175,14 +173,14 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
         uint4 af[NW][4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            af[0][t] = frag(s0, wm * 64 + 16 * t + l16);
+            af[0][t] = frag(s0, wave * 64 + 16 * t + l16);
             if constexpr (WDT == VGX_F16) widen_f16x8(af[0][t], af[0][t], af[NW - 1][t]);
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
-                const uint4 bf = frag(s0 + A_B + p * BH_B, wn * 64 + 16 * c + l16);
+                const uint4 bf = frag(s0 + A_B + p * BH_B, 16 * c + l16);
 #pragma unroll
                 for (int w = 0; w < NW; ++w)
 #pragma unroll
@@ -195,16 +193,15 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
     };
 
     const int nb = blk_hi - blk_lo;
-#pragma unroll
-    for (int s = 0; s < NS - 1; ++s) issue(blk_lo + s, s);
+    issue(blk_lo, 0);
     int cur = 0;
     for (int k = 0; k < nb; ++k) {
         // block k of this wave has landed and its reads of block k - 1 are done; the barrier extends both
         // to the workgroup, so block k is complete and the stage of block k - 1 is free
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NPW * (NS - 2)) : "memory");
-        issue(blk_lo + k + NS - 1, cur == 0 ? NS - 1 : cur - 1);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        issue(blk_lo + k + 1, cur ^ 1);
         compute(cur);
-        cur = cur + 1 == NS ? 0 : cur + 1;
+        cur ^= 1;
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the stages are free for the epilogue
 
@@ -214,7 +211,7 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
 #pragma unroll 1
         for (int e = 0; e < 16; ++e) {
             const int c = e >> 2, t = e & 3;
-            const int64_t b = b0 + wn * 64 + 16 * c + l16, crq = rq0 + wm * 16 + 4 * t + lg;
+            const int64_t b = b0 + 16 * c + l16, crq = rq0 + wave * 16 + 4 * t + lg;
             if (b >= batch || crq >= n_rq) continue;
             float *v = at(t, b, crq, c);
 #pragma unroll 1
@@ -226,11 +223,11 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
         bool bad = false;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const int64_t b = b0 + wn * 64 + 16 * c + l16;
+            const int64_t b = b0 + 16 * c + l16;
             if (b >= batch) continue;
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const int64_t crq = rq0 + wm * 16 + 4 * t + lg;
+                const int64_t crq = rq0 + wave * 16 + 4 * t + lg;
                 if (crq >= n_rq) continue;
                 float4 v;
                 v.x = acc[t][c][0]; v.y = acc[t][c][1]; v.z = acc[t][c][2]; v.w = acc[t][c][3];
@@ -248,9 +245,9 @@ __global__ __launch_bounds__(TM *TN / 64, TM *TN / 64 <= 256 ? 2 : 1) void wgemm
     float *et = reinterpret_cast<float *>(smem);
 #pragma unroll
     for (int half = 0; half < TM / 64; ++half) {
-        if (wm == half) {
+        if (wave == half) {
             bool bad = false;
-            auto at = [&](int t, int c) { return et + (wn * 64 + 16 * c + l16) * kERow + 16 * t + 4 * lg; };
+            auto at = [&](int t, int c) { return et + (16 * c + l16) * kERow + 16 * t + 4 * lg; };
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
