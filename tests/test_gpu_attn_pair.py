@@ -25,11 +25,12 @@ def _ref(q, runs):
 
 @pytest.mark.parametrize("H,G", [(4, 4), (4, 2), (8, 2), (12, 2), (16, 2)])
 @pytest.mark.parametrize("T,lens,ws", [(1, (319,), True), (17, (63, 65, 260), True), (129, (64, 1, 128), False),
-                                       (333, (257, 512), True), (65, (257, 62), False), (700, (), False), (1300, (64,), False)])
+                                       (333, (257, 512), True), (65, (257, 62), False), (700, (), False), (1300, (64,), False),
+                                       (700, (900,), True)])
 @pytest.mark.parametrize("kvdt", [torch.float32, torch.bfloat16])
 def test_prefill_tiles_match_oracle(dev, H, G, T, lens, ws, kvdt):
-    """Tile edges of 64 and 128 keys, 1 .. 1300 queries (narrow, wide, key ranges with a Workspace), every group size, both query
-    types; K and V rows at a stride of their own."""
+    """Tile edges of 64 and 128 keys, 1 .. 1300 queries (narrow, wide, key ranges with a Workspace over few and many keys),
+    every group size, both query types; K and V rows at a stride of their own."""
     rng = np.random.default_rng(H + 7 * T + sum(lens))
     runs = [tuple(_t(rng.standard_normal((G, n, 136)), kvdt)[:, :, :128] for _ in range(2)) for n in lens + (T,)]
     w = ops.Workspace(dev) if ws else None

@@ -819,15 +819,19 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_merge_kernel(Prefi
 // shares each staged tile: 12 query / 2 KV heads at L = 8192, bf16: 333 -> 295 us with 2 x 6 waves of 16 instead of
 // 6 of 32, -> 247 us with 128-key tiles by LDS DMA.  One and two heads per group take 8 and 4 waves per head: a
 // 1024-query chunk over 2560 keys at 4 / 4 heads, bf16, 127 -> 43 us, at 8 / 4 104 -> 48 us against the one-wave
-// workgroups that staged V through registers (fp32 planes: 331 -> 53 us for 777 queries over 1901 keys at 4 / 4).  Eight heads per
-// group keep 8 waves of 32 bf16 queries (16 waves would need <= 128 registers and spill).
+// workgroups that staged V through registers (fp32 planes, 1024 queries over 3584 keys at 4 / 4:
+// 597 -> 196).  Eight heads per group keep 8 waves of 32 bf16 queries (16 waves would need <= 128 registers and spill).
 // A launch of fewer workgroups than CUs takes half the waves per head (narrow), twice the workgroups.  With a
 // workspace the key ranges fill the CUs already, and the wide shape, which stages half the tiles per query, is ahead
-// while they do: the 1024-query bf16 chunk at 12 / 2 heads over 3584 keys (64 wide tiles x 4 ranges against 128 x 2)
-// 83 -> 68 us, 700 queries over 2236 (44 x 4) 56 -> 52; 400 (26) loses, 42 -> 50.  fp32 K / V with key ranges stay on
-// the in-place kernel and its shapes.
+// from 40 wide tiles on if there are keys enough.  bf16 chunks, wide | narrow, us: 12 / 2 heads 1024 queries (64
+// tiles) over 3584 keys 63.5 | 76.7, 2048 keys 47.8 | 51.5, their own 1024 keys 37.4 | 34.4; 700 (44) over 3260 60.4 |
+// 71.8, 1724 45.6 | 46.5, 700 35.2 | 29.0; 400 (26) 55.4 | 48.7, 41.5 | 37.1, 31.0 | 27.7.  Wide against narrow at 8 / 2,
+// 8 / 4, 16 / 4 and 8 / 8 heads: 44-64 tiles 0.77-0.81, 0.89-0.96, 1.05-1.26 for 2900-3600, 1400-2048 and 400-1024
+// keys; 16-32 tiles 1.03-1.08; 128 tiles 0.98 over 1024 keys.  fp32 K / V with key ranges stay on the in-place
+// kernel and its shapes.
 constexpr int kPrefillNarrowBelow = 256;
 constexpr int kSplitNarrowBelow = 40;
+constexpr int kSplitWideKeys = 1280, kSplitWideTiles = 128;   // keys, or wide tiles, from which the wide shape is ahead
 // Fewer keys than this in every block: the conversion's own launch costs more than the faster tiles give, and fp32
 // K / V are split by every workgroup.  Causal, that | planes, us: 100 keys 19.9 | -, 128 20.7 | 18.6, 200 30.2 | 23.7,
 // 512 61.9 | 42.8 at 12 / 2 heads; 128 keys at 4 / 4, 8 / 2, 16 / 2 heads 27.3 | 18.4, 19.2 | 17.4, 21.4 | 19.8.
@@ -874,9 +878,15 @@ PrefillPlan prefill_plan(int kv, const vgx_attn_block *blocks, int n_blocks, int
             if (blocks[i].n_q > 0) t += (blocks[i].n_q + q - 1) / q * G;
         return t;
     };
-    const int wide = kv == kKvF32 ? 32 : 16 * prefill_nqt(grp, kv) * prefill_qw(grp, kv, false);
-    p.narrow = prefill_qw(grp, kv, false) > 1 &&
-               count(wide) < (split && may_wide && kv != kKvF32 ? kSplitNarrowBelow : kPrefillNarrowBelow);
+    for (int i = 0; i < n_blocks; ++i) {
+        int64_t keys = 0;
+        for (int r = 0; blocks[i].n_q > 0 && r < blocks[i].n_runs; ++r) keys += blocks[i].runs[r].len;
+        p.max_keys = std::max(p.max_keys, keys);
+    }
+    const int64_t wide = count(kv == kKvF32 ? 32 : 16 * prefill_nqt(grp, kv) * prefill_qw(grp, kv, false));
+    const bool ranges_fill = split && may_wide && kv != kKvF32 && wide >= kSplitNarrowBelow &&
+                             (p.max_keys >= kSplitWideKeys || wide >= kSplitWideTiles);
+    p.narrow = prefill_qw(grp, kv, false) > 1 && wide < kPrefillNarrowBelow && !ranges_fill;
     p.qtile = 16 * prefill_nqt(grp, kv) * prefill_qw(grp, kv, p.narrow);   // queries per workgroup
     p.tiles = count(p.qtile);
     if (split && p.tiles > 0 && p.tiles < kPrefillNarrowBelow)
@@ -884,10 +894,8 @@ PrefillPlan prefill_plan(int kv, const vgx_attn_block *blocks, int n_blocks, int
     if (kv != kKvPlanes) return p;
     PlaneArgs &pa = p.planes;
     pa.G = (int)G;
-    for (int i = 0; i < n_blocks; ++i) {
-        int64_t keys = 0;
+    for (int i = 0; i < n_blocks; ++i)
         for (int r = 0; blocks[i].n_q > 0 && r < blocks[i].n_runs; ++r) {
-            keys += blocks[i].runs[r].len;
             const vgx_kv_run &R = blocks[i].runs[r];
             int u = 0;
             while (u < pa.n_runs && (pa.run[u].k != R.k || pa.run[u].v != R.v || pa.run[u].rstride != R.row_stride ||
@@ -903,8 +911,6 @@ PrefillPlan prefill_plan(int kv, const vgx_attn_block *blocks, int n_blocks, int
             pa.run[u].len = std::max(pa.run[u].len, R.len);
             p.run_of[i][r] = u;
         }
-        p.max_keys = std::max(p.max_keys, keys);
-    }
     for (int u = 0; u < pa.n_runs; ++u) {
         PlaneRun &n = pa.run[u];
         n.planes = reinterpret_cast<uint16_t *>(p.bytes);        // offsets; the call adds the workspace

@@ -556,7 +556,6 @@ def attn_prefill(blocks, H: int, G: int, scale: Optional[float] = None, ws: Opti
     ints: the bias row of head h, < 0: none) and ``bias_run``: query t of head h adds
     bias[t, bias_head_row[h], j] to its score with key j of that run.  With ``ws`` (a Workspace) a launch
     of few query tiles splits its keys over more workgroups (vgx_attn_prefill_ws)."""
-    lib = L.load()
     if not blocks:
         return
     D = blocks[0]["q"].shape[-1]
@@ -589,7 +588,8 @@ def attn_prefill(blocks, H: int, G: int, scale: Optional[float] = None, ws: Opti
                 ra[j] = L.KVRun(k.data_ptr(), v.data_ptr(), n, k.stride(1), k.stride(0))
                 keep.append((k, v))
                 keys += n
-            max_keys = max(max_keys, keys)
+            if keys > max_keys:
+                max_keys = keys
             arr[i] = L.AttnBlock(q.data_ptr(), q.stride(0), q.stride(1), out.data_ptr(), out.stride(0), out.stride(1),
                                  q.shape[0], int(b.get("causal_base", -1)), len(runs), ra)
             if b.get("bias") is not None:
