@@ -205,3 +205,29 @@ def test_prefill_workspace_sizes_one_head_per_group(dev, kvdt, T):
         assert (rc == 0) == (size >= full // 2 or T == 1024) and int((ws[size:] != 7).sum()) == 0
         if rc == 0:
             assert np.abs(out.double().cpu().numpy() - ref).max() <= (TOL32 if kvdt == torch.float32 else TOL)
+
+
+def test_prefill_planes_in_a_captured_graph(dev):
+    """A captured call with planes: replays, with eager calls over other keys between them, give the eager bits."""
+    rng = np.random.default_rng(13)
+    H, G, T = 12, 2, 300
+    sets = [tuple(_t(rng.standard_normal(s)) for s in ((T, H, 128), (G, T, 128), (G, T, 128))) for _ in range(3)]
+
+    def run(q, k, v, out):
+        ops.attn_prefill([{"q": q, "out": out, "runs": [(k, v)], "causal_base": 0}], H, G)
+        return out
+    eager = [run(*s, torch.empty(T, H, 128, device=dev)) for s in sets]
+    held, out = tuple(t.clone() for t in sets[0]), torch.zeros(T, H, 128, device=dev)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(*held, out)
+    for i in (0, 1, 2, 0):
+        for t, src in zip(held, sets[i]):
+            t.copy_(src)
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        other = run(*sets[(i + 1) % 3], torch.empty(T, H, 128, device=dev))
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager[i]) and torch.equal(other, eager[(i + 1) % 3]), f"replay of {i}"

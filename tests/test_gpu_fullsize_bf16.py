@@ -4,8 +4,8 @@ repo's VLT3 writer, loaded through the drop-in loader (ModelWeights.from_vlt3: v
 NaN / Inf scan, packing of the BF16 rows), decoding at 100K-token context against the reference C
 runtime (runtime/vault3.c, whose row_dot widens BF16 to fp32, :510-525) on the identical seeded state.
 Bars as for the hybrid-Q4_0 model: rel < 1e-4, max|dlogit| <= 5e-2, 100% top-1, identical
-segment-memory slots after the chunk boundary; batch 16 (the fp32 MFMA GEMM over BF16 weights,
-including the LM head) against the runtime stepping each sequence alone.
+segment-memory slots after the chunk boundary; batch 16 (the MFMA GEMM over BF16 weights with
+the activations in bf16 pieces, including the LM head) against the runtime stepping each sequence alone.
 """
 import os
 import tempfile

@@ -230,7 +230,7 @@ def test_gemv_fused_rmsnorm_equals_separate(dev, dt):
 @pytest.mark.parametrize("batch", [1, 3, 8, 40, 200])
 def test_plain16_swiglu_and_norm(dev, dt, batch):
     """BF16 / F16 gate/up with the fused SwiGLU, and the projections with an RMSNorm prologue, over the
-    GEMV (batch < 8) and the fp32 MFMA GEMM (batch >= 8, the norm applied by a separate launch)."""
+    GEMV (batch < 8) and the MFMA GEMM (batch >= 8, the norm applied by a separate launch)."""
     rows, cols = 512, 1536
     rng = np.random.default_rng(batch + dt)
     rg, ru = _blocks(dt, rows, cols, 1), _blocks(dt, rows, cols, 2)

@@ -89,9 +89,9 @@ def test_wgemm_leaves_the_tile_counters(dev, dt):
 @pytest.mark.parametrize("rows,cols,batch", [(70, 96, 9), (258, 1536, 70), (33000, 480, 9)])
 @pytest.mark.parametrize("swiglu", [False, True])
 def test_wgemm_infinities(dev, dt, rows, cols, batch, swiglu):
-    """Infinite and NaN weights and activations (the fp32 MFMA, several K ranges, one): against activations of few bits, whose lower
-    pieces are zero, against zeros, each other and ordinary elements.  An output is infinite or NaN where the float64
-    product is, and within the usual bound elsewhere."""
+    """Infinite and NaN weights and activations (the fp32 MFMA, several K ranges, one): against activations of few
+    bits, whose lower pieces are zero, against zeros, each other and ordinary elements.  An output is infinite or NaN
+    where the float64 product is, and within the usual bound elsewhere."""
     rng = np.random.default_rng(rows)
     td = torch.bfloat16 if dt == codec.BF16 else torch.float16
 
@@ -173,3 +173,32 @@ def test_qgemm_16bit_weights_without_the_planes(dev, dt, how, epi):
         out = ref[0] + (y0 if epi == L.EPI_ACCUM else 0.0)
         tol = bound[0] + np.abs(out) * 2e-7
     assert np.all(np.abs(y.double().cpu().numpy() - out) <= tol)
+
+
+@pytest.mark.parametrize("dt", [codec.BF16, codec.F16])
+@pytest.mark.parametrize("rows,cols,batch", [(1536, 8960, 16), (70, 800, 600)])
+def test_wgemm_in_a_captured_graph(dev, dt, rows, cols, batch):
+    """A captured call (down projection of a decode batch with K splits; one K range or few): its scratch belongs to the
+    graph, so replays with eager calls of other activations between them give the eager bits."""
+    rng = np.random.default_rng(rows)
+    w = ops.QWeight.from_blocks(dt, rows, cols, vlt3.quantize(dt, (rng.standard_normal((rows, cols)) * 0.05)
+                                                              .astype(np.float32)), dev)
+    xs = [torch.from_numpy(rng.standard_normal((batch, cols)).astype(np.float32)).to(dev) for _ in range(3)]
+    eager = [ops.qlinear(w, x) for x in xs]
+    x, out = xs[0].clone(), torch.zeros(batch, rows, device=dev)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        ops.qlinear(w, x, out=out)
+    torch.cuda.current_stream().wait_stream(s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ops.qlinear(w, x, out=out)
+    for i in (0, 1, 2, 0):
+        x.copy_(xs[i])
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        other = ops.qlinear(w, xs[(i + 1) % 3])
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager[i]) and torch.equal(other, eager[(i + 1) % 3]), f"replay of {i}"

@@ -663,12 +663,13 @@ __global__ __launch_bounds__(256, 3) void qgemm_tile_dma_kernel(const uint8_t *_
 
 // ---------------------------------------------------------------------------------------------
 // F32 weights (the segment scorer's fc1, F32 model files), and BF16 / F16 weights of few columns (wgemm_pays), of
-// callers without a workspace or past wgemm_tile_kernel's buffer ranges, for many activation rows, 16-bit elements widened exactly to fp32 as they are fetched: fp32 MFMA
-// (v_mfma_f32_16x16x4_f32), so products and sums stay fp32 as in the reference.  A workgroup of 4
+// callers without a workspace or past wgemm_tile_kernel's buffer ranges, for many activation rows, 16-bit
+// elements widened exactly to fp32 as they are fetched: fp32 MFMA (v_mfma_f32_16x16x4_f32), so products and sums
+// stay fp32 as in the reference.  A workgroup of 4
 // waves owns 64 weight rows x 64 activation rows (each wave 32 x 32 as 2 x 2 tiles); per 32-wide
 // block of K the workgroup stages both 64 x 32 fp32 tiles in LDS (double-buffered, one barrier per
 // block, next block's loads in flight during the current one's MFMAs).  Weights are read from the
-// packed row-quad layout (a row-quad block is 4 rows x 32 floats, contiguous).
+// packed row-quad layout (a row-quad block is 4 rows x 32 elements, contiguous).
 constexpr int kFT = 64;                   // rows of each operand per workgroup tile
 constexpr int kFRow = QK + 1;             // floats per staged row (one float of padding)
 
@@ -2532,9 +2533,9 @@ int vgx_qgemm(int dtype, const void *w_packed, int64_t rows, int64_t cols, const
     if (dtype == VGX_F32 || dtype == VGX_BF16 || dtype == VGX_F16) {
         if (norm_w) return VGX_E_ARG;                 // plain weights: no fused RMSNorm on this path
         // 16-bit weights on the 16-bit matrix cores where that pays, the caller brought the workspace and the
-        // operands fit the DMA's buffer ranges and 16-byte pieces; else (the workspace is optional here) on the fp32 MFMA.  Gate/up |
-        // down of BF16 files at 8, 40, 333, 1024 rows: 107 -> 25, 108 -> 33, 243 -> 76, 591 -> 184 us | 472 -> 24,
-        // 474 -> 28, 462 -> 53, 467 -> 107 us
+        // operands fit the DMA's buffer ranges and 16-byte pieces; else (the workspace is optional here) on the
+        // fp32 MFMA.  Gate/up | down of BF16 files at 8, 40, 333, 1024 rows: 107 -> 25, 108 -> 33, 243 -> 76,
+        // 591 -> 184 us | 472 -> 24, 474 -> 28, 462 -> 53, 467 -> 107 us
         const dim3 grid((unsigned)((n_rq + kFT / 4 - 1) / (kFT / 4)), (unsigned)((batch + kFT - 1) / kFT));
         if (dtype != VGX_F32 && wgemm_pays(dtype, nblk, (int64_t)grid.x * grid.y, batch) && workspace &&
             (uintptr_t)workspace % 256 == 0 && (uintptr_t)w_packed % 16 == 0 &&
