@@ -23,7 +23,8 @@ pytestmark = pytest.mark.gpu
 def test_wgemm_matches_oracle(dev, dt, rows, cols, batch, epi):
     """Tile edges (256 weight rows, 64 activation rows), one K block, K splits with a short last one, every
     epilogue, both sides of the line to the fp32 MFMA (few columns); "edge": weights and rows of extreme
-    magnitudes (fp16 subnormals, rows of 1e-30 .. 1e30) and non-finite activations; "strided": rows at an odd float offset and stride."""
+    magnitudes (fp16 subnormals, rows of 1e-30 .. 1e30) and non-finite activations; "strided": rows at an odd
+    float offset and stride."""
     rng = np.random.default_rng(rows + cols + batch)
     mk = lambda seed: vlt3.quantize(dt, np.random.default_rng(seed).standard_normal((rows, cols)).astype(np.float32)
                                     * (1e-5 if epi == "edge" else 0.05))  # noqa: E731
@@ -145,8 +146,8 @@ def test_wgemm_elements_keep_their_own_exponent(dev, dt, big):
 @pytest.mark.parametrize("how", ["none", "short", "weights at 8 bytes"])
 @pytest.mark.parametrize("epi", [L.EPI_STORE, L.EPI_ACCUM, L.EPI_SWIGLU])
 def test_qgemm_16bit_weights_without_the_planes(dev, dt, how, epi):
-    """vgx_qgemm of 16-bit weights where the DMA tiles cannot run (no workspace, one without room for the partials, weights that are
-    not 16-byte aligned) runs on the fp32 MFMA: odd row counts, more rows and activations than a tile."""
+    """vgx_qgemm of 16-bit weights where the DMA tiles cannot run (no workspace, one without room for the partials,
+    weights that are not 16-byte aligned) runs on the fp32 MFMA: odd row counts, more rows and activations than a tile."""
     lib, rng = L.load(), np.random.default_rng(4)
     rows, cols, batch = (106 if epi == L.EPI_SWIGLU else 205), 1056, 70
     mk = lambda: vlt3.quantize(dt, (rng.standard_normal((rows, cols)) * 0.05).astype(np.float32))  # noqa: E731

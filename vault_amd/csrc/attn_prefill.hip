@@ -35,9 +35,9 @@
 // staged by LDS DMA; without it, for few keys, or with key ranges (vgx_attn_prefill_ws) every workgroup loads
 // its fp32 tiles into registers during the previous tile's math, splits them and stores the planes into LDS, K as
 // is (padded rows), V transposed: the same pieces in the same order, so the same bits: two sequences
-// of 2500 at 12 / 2 heads 349 -> 255 us for the whole call, 1024 queries over 3584 keys at 4 / 4 heads 597 -> 196.  Six
-// products of 64.6 million pairs x 128 dims x 2 are 198 GFLOP there, 165 us at the 1.2 PFLOP/s of a large bf16
-// product on this card; 25 us are the planes and the sinks.  What it took beside the DMA: each wave's loads of a
+// of 2500 at 12 / 2 heads 349 -> 253 us for the whole call, 1024 queries over 3584 keys at 4 / 4 heads 597 -> 196.  Six
+// piece products of the 33 GFLOP there are 198 GFLOP, 165 us at the 1.2 PFLOP/s of a large bf16 product on
+// this card; 25 us are the planes and the sinks.  What it took beside the DMA: each wave's loads of a
 // tile a fixed set of a few instructions (272 -> 255 us; at four waves a workgroup 255 -> 196), the operands of the next
 // 32 dims read while this one's are multiplied (266 -> 255, 229 -> 196).
 // In both products a lane of the 16 x 16 output owns
@@ -815,12 +815,13 @@ __global__ __launch_bounds__(64 * GRP * QW) void attn_prefill_merge_kernel(Prefi
 }
 
 // Launch shape per K / V kind and heads per group: QW waves of NQT 16-query tiles per head.  Waves of 16 queries
-// (at most 168 registers: three per SIMD) beat waves of 32 (226-256 registers, two), and a workgroup of 8-12 waves
-// shares each staged tile: 12 query / 2 KV heads at L = 8192, bf16: 333 -> 295 us with 2 x 6 waves of 16 instead of
-// 6 of 32, -> 247 us with 128-key tiles by LDS DMA.  One and two heads per group take 8 and 4 waves per head: a
-// 1024-query chunk over 2560 keys at 4 / 4 heads, bf16, 127 -> 43 us, at 8 / 4 104 -> 48 us against the one-wave
-// workgroups that staged V through registers (fp32 planes, 1024 queries over 3584 keys at 4 / 4:
-// 597 -> 196).  Eight heads per group keep 8 waves of 32 bf16 queries (16 waves would need <= 128 registers and spill).
+// (at most 168 registers: three per SIMD at 6 heads per group, where 12 waves share the one workgroup that the LDS
+// holds; two at the others) beat waves of 32 (226-256 registers), and a workgroup of 8-12 waves shares each
+// staged tile: 12 query / 2 KV heads at L = 8192, bf16: 333 -> 295 us with 2 x 6 waves of 16 instead of 6 of 32,
+// -> 247 us with 128-key tiles by LDS DMA.  One and two heads per group take 8 and 4 waves per head: a 1024-query
+// chunk over 2560 keys at 4 / 4 heads, bf16, 127 -> 43 us, at 8 / 4 104 -> 48 us against the one-wave workgroups
+// that staged V through registers (fp32 planes, 1024 queries over 3584 keys at 4 / 4: 597 -> 196).  Eight heads
+// per group keep 8 waves of 32 bf16 queries (16 waves would need <= 128 registers and spill).
 // A launch of fewer workgroups than CUs takes half the waves per head (narrow), twice the workgroups.  With a
 // workspace the key ranges fill the CUs already, and the wide shape, which stages half the tiles per query, is ahead
 // from 40 wide tiles on if there are keys enough.  bf16 chunks, wide | narrow, us: 12 / 2 heads 1024 queries (64
